@@ -547,6 +547,60 @@ int dispatch_gemm(int bits, int cb, const GemmArgs& g, hipStream_t s)
     return -1;
 }
 
+int dispatch_rows(int bits, int cb, const RowsArgs& g, hipStream_t s)
+{
+    switch (bits)
+    {
+        case 1: return exl3k_rows_k1(g, cb, s);
+        case 2: return exl3k_rows_k2(g, cb, s);
+        case 3: return exl3k_rows_k3(g, cb, s);
+        case 4: return exl3k_rows_k4(g, cb, s);
+        case 5: return exl3k_rows_k5(g, cb, s);
+        case 6: return exl3k_rows_k6(g, cb, s);
+        case 7: return exl3k_rows_k7(g, cb, s);
+        case 8: return exl3k_rows_k8(g, cb, s);
+        case 17: return exl3k_rows_k17(g, cb, s);
+        case 18: return exl3k_rows_k18(g, cb, s);
+        case 19: return exl3k_rows_k19(g, cb, s);
+    }
+    return -1;
+}
+
+// Row tiles and k split of the row-tile GEMM (exl3_rows.hip).  As few row tiles as 128 rows allow,
+// equal in height.  The k split S minimises this model (us, fitted on MI355X over K = 3 / 4, nine
+// shapes from 4096 x 1024 to 8192 x 28672 and S = 1..32; within ~10 %):
+//   rounds of workgroups over the CUs x units per k half (128 k each) x the unit's time, which the
+//   decode sets and the row groups add to; the fill and the epilogue once per round (twice as
+//   many workgroups share a CU up to 4 groups); the last arrival's sum of S partials per group.
+// Returns the model's time, input rotation included.
+double rows_plan(const Workspace& w, int m, int k, int n, RowsArgs& g)
+{
+    static const double unit_us[9] = { 0.0, 0.94, 0.94, 1.04, 1.06, 1.13, 1.2, 0.0, 1.32 };
+    const int chunks = n / 128, blocks = k / 128, nt = (m + 127) / 128;
+    int R = ((m + nt - 1) / nt + 15) / 16;
+    if (R == 7) R = 8;
+    const long tiles = (long) nt * chunks;
+    const size_t part1 = (size_t) tiles * R * 16 * 128 * sizeof(float);
+    double best = 0.0;
+    int S = 0;
+    for (int sp = 1; sp <= 64 && sp <= blocks; ++sp)
+    {
+        if (sp > 1 && part1 * sp > w.partial_bytes) break;
+        const long rounds = (tiles * sp + w.num_cus - 1) / w.num_cus;
+        const int units = (blocks + sp - 1) / sp;
+        const double t = 4.0 + rounds * units * unit_us[R] + (R <= 4 ? (rounds + 1) / 2 : rounds) * (5.5 + 0.9 * R)
+                       + (sp > 1 ? 0.12 * R * sp : 0.0);
+        if (!S || t < best) { best = t; S = sp; }
+    }
+    g.groups = R;
+    g.splits = S;
+    g.part = w.partials;
+    g.ctr = w.counters;
+    g.xcd = w.num_xcd > 0 && w.alarm && chunks % w.num_xcd == 0 && (size_t) tiles * 32 <= w.counter_ints / 2 ? w.num_xcd : 0;
+    g.xg = xcd_guard(w.alarm);
+    return best;
+}
+
 int dispatch_gemv(int bits, int cb, const GemvArgs& g, hipStream_t s)
 {
     switch (bits)
@@ -940,13 +994,16 @@ int gemm_impl(const Workspace* ws, const uint16_t* A, const uint16_t* trellis, v
         if (rc) return hip_fail(rc, name);
     }
     const uint16_t* A_rot = suh ? A_had : A;
-    // Medium batches: the row-batched matrix-core GEMV in 16-row groups when it beats the tiled
-    // GEMM.  Measured on MI355X (K = 2..4, k x n from 4096 x 1024 to 17408 x 5120, m = 16..192):
-    // a 16-row group takes ~8 us + 0.37 ns per 1000 weights; a GEMM round (up to one tile per CU)
-    // ~28 ns per k; with the split k, ~27 us + 28 ns per k of a split (input rotation, the
-    // partial tiles and the fixup included).  The groups win at 16 rows, break even at 24-32.
+    // More than 8 rows: the row-tile GEMM (exl3_rows.hip), the tiled GEMM or, up to 16 rows, the
+    // matrix-core GEMV, whichever its time model puts first (us, input rotation included).  Measured
+    // on MI355X (K = 4 3INST, row tiles / tiled GEMM): 4096 x 14336 at 33 / 100 / 256 rows 27 / 38 /
+    // 59 against 52 / 56 / 66, 17408 x 5120 37 / 52 / 87 against 68 / 71 / 83, 8192 x 28672 80 / 97
+    // / 209 against 152 / 154 / 174: row tiles up to ~128-250 rows, the tiled GEMM above.
+    //   tiled GEMM: 22 us + 30 ns per k of a round (of a split), and with the split k 0.25 us per MB
+    //   of partial tiles; GEMV group: 8 us + 0.37 ns per 1000 weights.
     // force_shape_idx 1 takes the GEMV for any row count (16-row groups, each split in two
-    // launches of at most 8 rows when the matrix-core GEMV is off or its plan does not fit).
+    // launches of at most 8 rows when the matrix-core GEMV is off or its plan does not fit), 2 the
+    // tiled GEMM.
     // The tiled GEMM splits k when its tiles fill at most half the CUs (LDS-DMA form): S ranges per
     // tile, as many as fill the CUs, at least 4 stages of 32 k each, the S fp32 partial tiles
     // within the workspace; the fixup kernel sums them in k order and runs the epilogue.
@@ -964,9 +1021,21 @@ int gemm_impl(const Workspace* ws, const uint16_t* A, const uint16_t* trellis, v
     if (force_shape_idx == 0 && gemv_mfma_mode() != 0)
     {
         const long rounds = (blocks + ws->num_cus - 1) / ws->num_cus;
-        const double t_groups = ((m + 15) / 16) * (8.0 + 3.7e-7 * (double) n * k);
-        const double t_gemm = splits > 1 ? 27.0 + 0.028 * k / splits : 0.028 * k * rounds;
-        groups = t_groups < t_gemm;
+        const double t_gemm = 22.0 + (splits > 1 ? 0.030 * k / splits + 1e-6 * splits * (double) m * n : 0.030 * k * rounds);
+        const double t_group = m <= 16 ? 8.0 + 3.7e-7 * (double) n * k : 1e30;
+        RowsArgs rr;
+        memset(&rr, 0, sizeof(rr));
+        rr.A_rot = A_rot;
+        rr.trellis = trellis; rr.C = C; rr.svh = svh;
+        rr.m = m; rr.k = k; rr.n = n; rr.c_fp32 = c_fp32 ? 1 : 0;
+        const double t_rows = rows_plan(*ws, m, k, n, rr);
+        if (staging == 0 && t_rows <= t_gemm && t_rows <= t_group)
+        {
+            int rc = dispatch_rows(bits, cb, rr, s);
+            if (rc) return hip_fail(rc, name);
+            return m <= 16 ? EXL3_AMD_TAG_GEMV : EXL3_AMD_TAG_GEMM;
+        }
+        groups = t_group <= t_gemm;
     }
     if (groups)
     {

@@ -497,7 +497,40 @@ void dense_split_fixup(const float* __restrict__ part, void* __restrict__ C, con
     gemm_store(v0, v1, C, c_fp32, has_svh, svp, (size_t) row * ldc + c0 + 2 * lane, lane);
 }
 
+// The row-tile GEMM's k ranges without the hand-off (exl3_rows.hip): one wave per (row tile,
+// chunk, row) adds the ranges in k order, rotates and stores.
+__global__ __launch_bounds__(256)
+void rows_finish(const RowsArgs g)
+{
+    const int lane = threadIdx.x & 63, chunks = g.n / 128, RT = 16 * g.groups;
+    const long job = (long) blockIdx.x * 4 + (threadIdx.x >> 6);  // (row, chunk)
+    if (job >= (long) g.m * chunks) return;
+    const int row = (int) (job / chunks), chunk = (int) (job % chunks);
+    const size_t tile = (size_t) (row / RT) * chunks + chunk;
+    const float* p = g.part + (tile * g.splits * RT + row % RT) * 128 + 2 * lane;
+    float v0 = 0.0f, v1 = 0.0f;
+    for (int q0 = 0; q0 < g.splits; q0 += 4)
+    {
+        f32x2 v[4];
+        #pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = __builtin_nontemporal_load((const f32x2*) (p + (size_t) min(q0 + q, g.splits - 1) * RT * 128));
+        #pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (q0 + q < g.splits) { v0 += v[q].x; v1 += v[q].y; }
+    }
+    const bool has_svh = g.svh != nullptr;
+    const uint32_t svp = has_svh ? *(const uint32_t*) (g.svh + chunk * 128 + 2 * lane) : 0u;
+    gemm_store(v0, v1, g.C, g.c_fp32, has_svh, svp, (size_t) row * g.n + chunk * 128 + 2 * lane, lane);
+}
+
 }  // namespace
+
+int exl3k_rows_finish(const RowsArgs& g, hipStream_t s)
+{
+    const long jobs = (long) g.m * (g.n / 128);
+    hipLaunchKernelGGL(rows_finish, dim3((unsigned) ((jobs + 3) / 4)), dim3(256), 0, s, g);
+    return (int) hipGetLastError();
+}
 
 int exl3k_dense_gemm(const uint16_t* A, const uint16_t* WT, void* C, int c_fp32, const uint16_t* svh,
                      int m, int k, int n, int a_slabs, int w_slabs, int ldc, int variant, int cus,

@@ -168,6 +168,36 @@ int exl3k_gemm_k17(const GemmArgs& g, int cb, hipStream_t s);   // half rates 1.
 int exl3k_gemm_k18(const GemmArgs& g, int cb, hipStream_t s);
 int exl3k_gemm_k19(const GemmArgs& g, int cb, hipStream_t s);
 
+// Row-tile GEMM (exl3_rows.hip): C = A_rot @ W_hat (rotated by svh) in row tiles of 16 groups rows.
+struct RowsArgs
+{
+    const uint16_t* A_rot;      // (m, k) fp16: had(A o suh) or A itself
+    const uint16_t* trellis;    // (k/16, n/16, 16K) uint16
+    void* C;                    // (m, n) fp16 or fp32
+    const uint16_t* svh;        // (n) fp16 or null
+    int m, k, n;
+    int c_fp32;
+    int groups;                 // 16-row groups per row tile: 1..6 or 8
+    int splits;                 // k ranges per (row tile, 128-column chunk), at most k / 128
+    int xcd;                    // > 0: XCD-local hand-off (n / 128 a multiple of it); 0: rows_finish
+    float* part;                // splits > 1: (row tiles x chunks) x splits x 16 groups x 128 fp32
+    int* ctr;                   // xcd: zeroed counters, one 128-byte line per (row tile, chunk)
+    XcdGuard xg;
+};
+
+int exl3k_rows_k1(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k2(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k3(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k4(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k5(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k6(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k7(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k8(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k17(const RowsArgs& g, int cb, hipStream_t s);   // half rates 1.5 / 2.5 / 3.5: mul1
+int exl3k_rows_k18(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_k19(const RowsArgs& g, int cb, hipStream_t s);
+int exl3k_rows_finish(const RowsArgs& g, hipStream_t s);        // exl3_dense.hip
+
 // Grouped GEMM of the token-sorted MoE: one launch runs every row tile of one bitrate.  A row
 // tile is (expert, first row, rows <= 256) of the compacted row pool; workgroup b runs column
 // block b % nbn of list entry (b / nbn) / mats of matrix set (b / nbn) % mats and exits when the

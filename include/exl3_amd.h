@@ -33,7 +33,8 @@ extern "C" {
 #define EXL3_AMD_EHIP         -3   /* HIP runtime error                                     */
 #define EXL3_AMD_ENOMEM       -4   /* workspace allocation failed                           */
 
-/* Kernel tags returned by exl3_amd_gemm (the reference returns a shape index, 90 = GEMV). */
+/* Kernel tags returned by exl3_amd_gemm (the reference returns a shape index, 90 = GEMV): GEMV for
+ * the GEMV kernels and for one 16-row tile of the row-tile GEMM, GEMM for everything taller. */
 #define EXL3_AMD_TAG_GEMV     90
 #define EXL3_AMD_TAG_GEMM     91
 
