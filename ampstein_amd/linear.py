@@ -11,6 +11,9 @@ once is an error, and a half-integer K without mul1 is rejected (models.uc:46-66
 
 forward(x): more than RECON_ROWS rows and at most RECON_MAX_N output features go through
 exl3_gemm_recon; everything else through exl3_gemm into a fresh fp16 output; then + bias.
+RECON_ROWS is this build's line, not the engine's 144 (models.uc:35): below 2048 rows both routes
+rotate x to fp16, multiply the same fp16 weights in fp32 and rotate the sums, so the line moves
+no rounding point, only the time.
 """
 from __future__ import annotations
 
@@ -21,8 +24,13 @@ import torch
 from . import bundles, ops
 from .weights import Weights
 
-RECON_ROWS = 144       # models.uc:35
-RECON_MAX_N = 32768    # models.uc:36
+# exl3_gemm / exl3_gemm_recon on MI355X, us: 4096 -> 4096 at 145 / 256 / 512 rows 25 / 33 / 46
+# against 57 / 65 / 58, 14336 -> 4096 49 / 62 / 99 against 82 / 92 / 107, 8192 -> 28672 157 / 174 /
+# 296 against 250 / 246 / 324; at 768 rows of 17408 -> 5120 196 against 186, 8192 -> 28672 559
+# against 512.  exl3_gemm also needs no k x n fp16 buffer.
+RECON_ROWS = 512
+ENGINE_RECON_ROWS = 144   # models.uc:35
+RECON_MAX_N = 32768       # models.uc:36
 
 
 class LinearError(ValueError):
@@ -60,6 +68,13 @@ class LinearEXL3:
             out = ops.exl3_gemm_recon(x.contiguous(), self.trellis, self.suh, self.svh, self.K,
                                       self.mul1, self.mcg)
         else:
+            if m > ENGINE_RECON_ROWS:
+                # the engine's recon range: its input checks, and x in any strides
+                ops._need(x.dim() == 2 and x.size(1) == self.in_features and self.suh.numel() == self.in_features
+                          and self.svh.numel() == self.out_features,
+                          f"LinearEXL3: incompatible shapes (x {tuple(x.shape)}, weight {self.in_features} x "
+                          f"{self.out_features})")
+                x = x.contiguous()
             # exl3_gemm writes every element: no zero fill.  The binding hands the kernel a
             # scratch buffer of x's shape for the rotated input (amp_torch.cpp:11251-11294).
             out = torch.empty((m, self.out_features), dtype=torch.float16, device=x.device)

@@ -134,3 +134,25 @@ def test_linear_forward(tmp_path, orc, rows, K, cb, with_bias):
     err = np.abs(y - ref).max() / np.abs(ref).max()
     print(f"linear forward rows={rows} K={K} cb={cb} bias={with_bias}: rel err {err:.2e}", flush=True)
     assert err < 2e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [144, 145, 512, 513])
+def test_linear_forward_route_line(tmp_path, orc, rows):
+    """Around the engine's and this build's line between exl3_gemm and the recon route: x in any
+    strides from 145 rows on, and other ranks refused there."""
+    from ampstein_amd import _lib
+    from ampstein_amd.linear import LinearEXL3
+    k, n = 256, 384
+    L = synth.layer(k, n, 4, 0, seed=60 + rows)
+    _write_model(str(tmp_path), _layer_tensors("blk.o", L), False)
+    lin = LinearEXL3(open_weights(str(tmp_path)), "blk.o", 0)
+    x = synth.activations(rows, k, seed=rows)
+    xs = torch.from_numpy(x).cuda()
+    if rows > 144:
+        xs = torch.cat([xs, xs], 1)[:, :k]                 # rows 2 k apart
+        with pytest.raises(_lib.Exl3Error):
+            lin(xs.view(rows, 1, k) if xs.is_contiguous() else xs.contiguous().view(rows, 1, k))
+    y = lin(xs).float().cpu().numpy().astype(np.float64)
+    ref = orc.linear_f64(x, L.trellis, L.suh, L.svh, 4, cb=0)
+    assert np.abs(y - ref).max() / np.abs(ref).max() < 2e-3
