@@ -324,7 +324,6 @@ int gemv_mfma_mode()
 }
 
 // Work-split constants of the GEMV planner (measured on MI355X; see the comments at their uses).
-constexpr int GEMVM_TARGET_WG_PER_CU_X2 = 3;     // matrix-core GEMV: 1.5 workgroups per CU
 constexpr int GEMVM_STAGED_X_BYTES = 48 * 1024;  // its staged input rows, per workgroup
 constexpr int GEMV_LDS_WG_PER_CU = 4;            // LDS / stream kernels: 4 workgroups per CU
 
@@ -338,31 +337,33 @@ int gemv_plan(int m, int k, int n, int bszm, int num_cus, GemvArgs& g, size_t pa
         const bool use = m <= 16 && (m >= 2 ? mode != 0 : mode >= 2);
         if (use)
         {
-            const int KS = k / 16, chunks = n / 128;
+            const int blocks = k / 128, chunks = n / 128;
             const int mt = m == 1 ? 1 : (m <= 4 ? 4 : (m <= 8 ? 8 : 16));
-            // target grid: 1.5 workgroups per CU
-            const long target = (long) GEMVM_TARGET_WG_PER_CU_X2 * num_cus / 2;
-            // SB: k-tiles per workgroup, a multiple of 8 dividing k/16, at most 64 (16 units per
-            // wave; 32 for 16 rows); the largest whose grid still reaches the target (else the smallest), within
-            // 48 KB of staged input and the workspace.  Measured on MI355X over SB (Qwen 5120 x
-            // {5120, 17408}, 17408 x 5120, m = 1..16): the optimum sits at 1.5-2.7 workgroups per
-            // CU with SB 32-64; SB 8 (the most workgroups) is up to 1.5x slower.
-            int best = -1;
-            const int sb_max = mt >= 16 ? 32 : 64;                // 16 rows: SB 32 measured best
-            for (int d = 8; d <= KS && d <= sb_max; d += 8)
+            // k ranges S (of whole 128-row chunks, as equal as they come) per column chunk: the one that
+            // minimises this model (us, fitted on MI355X over S = 1..40 and m = 2..16 on seven Qwen-
+            // and Llama-shaped matrices; within ~10 %): the workgroups of the fullest CU x the mean
+            // of the average and the longest range x a 128-row chunk's time (decode, and the rows'
+            // rotation; a workgroup alone on its CU hides less: 1.65), 0.5 us per workgroup, and
+            // with S > 1 the hand-off and the last arrival's sum.  Ranges need not divide k evenly:
+            // 5120 x 5120 at 8 rows takes S = 12 (480 workgroups), 13.9 us with S = 10 before.
+            int best = 0;
+            double best_t = 0.0;
+            for (int sp = 1; sp <= blocks; ++sp)
             {
-                if (KS % d) continue;
-                if ((size_t) mt * (d * 16 + 4) * 4 > (size_t) GEMVM_STAGED_X_BYTES) break;
-                if ((size_t) (KS / d) * bszm * m * n * 4 > partial_bytes && KS / d > 1) continue;
-                if ((long) bszm * chunks * (KS / d) >= target || best < 0) best = d;
-                if ((long) bszm * chunks * (KS / d) < target) break;
+                const int nk = (blocks + sp - 1) / sp;           // 128-row chunks of the longest range
+                if ((size_t) mt * (nk * 128 + 4) * 4 > (size_t) GEMVM_STAGED_X_BYTES) continue;
+                if ((size_t) sp * bszm * m * n * 4 > partial_bytes && sp > 1) break;
+                const long per = ((long) bszm * chunks * sp + num_cus - 1) / num_cus;     // workgroups of a CU
+                const double t = 2.0 + per * 0.5 * ((double) blocks / sp + nk) * (0.5 + 0.027 * m) * (per == 1 ? 1.65 : 1.0) + 0.5 * per
+                         + (sp > 1 ? 1.5 + 0.02 * m * sp : 0.0);
+                if (!best || t < best_t) { best = sp; best_t = t; }
             }
             if (best > 0)
             {
                 g.stream_m1 = 0;
                 g.mfma_rows = 1;
-                g.slices_per_block = best;
-                g.slots = KS / best;
+                g.slices_per_block = 8 * ((blocks + best - 1) / best);
+                g.slots = best;
                 g.xs_chunks = 0;
                 return 0;
             }
@@ -389,6 +390,9 @@ int gemv_plan(int m, int k, int n, int bszm, int num_cus, GemvArgs& g, size_t pa
         if (best < 0 || (long) bszm * chunks * (KS / best) > target) best = d;   // fewest blocks >= target
         if ((long) bszm * chunks * (KS / d) <= target) break;
     }
+    // at least 3 workgroups per CU with whole columns (a vocabulary head): no split, so no hand-off
+    // or finish kernel (4096 -> 128256 at 6 bits: 98 us against 107 in two ranges)
+    const bool whole = stream && (long) bszm * chunks >= 3L * num_cus && ok_sb(KS);
     // M = 1 stream: 4 k-slices per wave below k = 8192, 16 from there: the best splits measured
     // on MI355X for the Llama-3-8B shapes in a captured sweep (4096 x 4096: 6.85 -> 6.45 us, the
     // sliced q/k/v bundle 9.1 -> 7.9 us against 8 per wave; 14336 x 4096 best at 16)
@@ -401,6 +405,7 @@ int gemv_plan(int m, int k, int n, int bszm, int num_cus, GemvArgs& g, size_t pa
         while (ok_sb(2 * pref) && (long) bszm * chunks * (KS / pref) > 8L * num_cus) pref *= 2;
         for (int d = pref; d >= 4; d /= 2)
             if (ok_sb(d) && ((size_t) (KS / d) * bszm * m * n * 4 <= partial_bytes || KS / d == 1)) { best = d; break; }
+        if (whole) best = KS;
         // policy EXL3_AMD_POLICY_GEMV_SLICES: a forced split (k-slices per workgroup) when valid
         const int forced = policy(EXL3_AMD_POLICY_GEMV_SLICES);
         if (forced > 0 && ok_sb(forced) && ((size_t) (KS / forced) * bszm * m * n * 4 <= partial_bytes || KS / forced == 1))

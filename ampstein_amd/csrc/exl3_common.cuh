@@ -344,6 +344,33 @@ __device__ __forceinline__ void fwht128_wave(float& v0, float& v1, int lane)
     fwht_stage<32>(v0, v1, lane);
 }
 
+// Hadamard-128 with 16 lanes per 128-vector, lane g of 16 holding elements 8 g .. 8 g + 7 (four
+// vectors per wave): widths 1, 2, 4 in-lane, then 8, 16, 32, 64 across lanes.  The stages and their
+// rounding are fwht128_wave's, so the results are the same bits.
+__device__ __forceinline__ void fwht128_lane8(float* e, int lane)
+{
+    #pragma unroll
+    for (int w = 1; w < 8; w <<= 1)
+    {
+        #pragma unroll
+        for (int i = 0; i < 8; ++i)
+        {
+            if (i & w) continue;
+            const float a = e[i], b = e[i + w];
+            e[i] = a + b;
+            e[i + w] = a - b;
+        }
+    }
+    #pragma unroll
+    for (int i = 0; i < 8; i += 2) fwht_stage<1>(e[i], e[i + 1], lane);
+    #pragma unroll
+    for (int i = 0; i < 8; i += 2) fwht_stage<2>(e[i], e[i + 1], lane);
+    #pragma unroll
+    for (int i = 0; i < 8; i += 2) fwht_stage<4>(e[i], e[i + 1], lane);
+    #pragma unroll
+    for (int i = 0; i < 8; i += 2) fwht_stage<8>(e[i], e[i + 1], lane);
+}
+
 // Output rotation of one fp32 row chunk (elements 2l, 2l+1) and store: had_fh / had_ff.
 __device__ __forceinline__ void gemm_store(float v0, float v1, void* C, int c_fp32, bool has_svh, uint32_t svp,
                                            size_t idx, int lane)

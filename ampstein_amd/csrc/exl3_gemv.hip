@@ -339,6 +339,9 @@ __device__ void weighted_reduce(const GemvArgs& g, int chunk, bool via_l2)
 // this workgroup's slot; in XCD mode the last workgroup of the (slot j, chunk) pair then sums
 // the partials -- in a fixed order -- rotates and stores.  Weighted mode adds a second hand-off
 // per chunk over all slots, whose last arrival runs the token-group reduction.
+// WIDE (the matrix-core rows): the sum with more loads in flight, and the registers for them; the
+// other kernels' register floor is set by this call (5 more cost gemv1_kernel a wave per SIMD).
+template <bool WIDE>
 __device__ void block_epilogue(const GemvArgs& g, const MatView& v, int j, int chunk, int slot, int splits,
                                const float* res, float* tmp, int* flag, uint32_t svp, int rs = 128)
 {
@@ -354,6 +357,46 @@ __device__ void block_epilogue(const GemvArgs& g, const MatView& v, int j, int c
         GEMV_STAMP(g, 4, 0);
         if (!arrive_last(g.xg, g.counters + ((size_t) j * chunks + chunk) * 32, splits, flag)) return;
         GEMV_STAMP(g, 6, *flag);
+        if (WIDE && m >= GEMV_WAVES)
+        {
+            // a wave sums, rotates and stores its rows two at a time, 8 slots' loads of each in
+            // flight, no LDS and no barrier (a thread per column pair, its pairs in turn, took 7.8 us
+            // for 8 rows of 40 slots)
+            for (int r0 = wave; r0 < m; r0 += 2 * GEMV_WAVES)
+            {
+                const int r1 = r0 + GEMV_WAVES;
+                const bool two = r1 < m;
+                float a0 = 0.0f, a1 = 0.0f, b0 = 0.0f, b1 = 0.0f;
+                for (int sp0 = 0; sp0 < splits; sp0 += 8)
+                {
+                    f32x2 va[8], vb[8];
+                    #pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        va[u] = load_l2_f32x2(pbase + ((size_t) min(sp0 + u, splits - 1) * m + r0) * 128 + 2 * lane);
+                    if (two)
+                    {
+                        #pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            vb[u] = load_l2_f32x2(pbase + ((size_t) min(sp0 + u, splits - 1) * m + r1) * 128 + 2 * lane);
+                        #pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            if (sp0 + u < splits) { b0 += vb[u].x; b1 += vb[u].y; }
+                    }
+                    #pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (sp0 + u < splits) { a0 += va[u].x; a1 += va[u].y; }
+                }
+                const size_t col = chunk * 128 + 2 * lane;
+                res_store(g, r0, chunk, lane,
+                          store_output(a0, a1, v.C, g.c_fp32, v.svh != nullptr, svp, (size_t) r0 * v.stride + col, lane, v.scale));
+                if (two)
+                    res_store(g, r1, chunk, lane,
+                              store_output(b0, b1, v.C, g.c_fp32, v.svh != nullptr, svp, (size_t) r1 * v.stride + col, lane, v.scale));
+            }
+            GEMV_STAMP(g, 7, 0);
+        }
+        else
+        {
         // sum the slots: threads split into G groups over the m * 64 column pairs; group gi takes
         // slots gi, gi + G, ...; the groups then combine in order through LDS
         const int pairs = m * 64;
@@ -392,6 +435,7 @@ __device__ void block_epilogue(const GemvArgs& g, const MatView& v, int j, int c
             const int col = chunk * 128 + 2 * lane;
             res_store(g, r, chunk, lane,
                       store_output(s0, s1, v.C, g.c_fp32, v.svh != nullptr, svp, (size_t) r * v.stride + col, lane, v.scale));
+        }
         }
     }
     else
@@ -705,7 +749,7 @@ void gemv_kernel(const GemvArgs g)
         res[r * 128 + 2 * lane + 1] = r0[nr][1];
     }
     __syncthreads();
-    block_epilogue(g, v, j, chunk, slot, splits, res, red, &flag, svp);
+    block_epilogue<false>(g, v, j, chunk, slot, splits, res, red, &flag, svp);
 }
 
 // Sum the split partials of each (slot, column chunk) in slot order, output rotation, store.
@@ -880,6 +924,10 @@ void gemv1_kernel(const GemvArgs g)
     __shared__ __align__(16) uint32_t xdup[GEMV_WAVES][2][128];
     __shared__ __align__(16) uint32_t xzero[GEMV_WAVES][128];
     *(u32x2*) &xzero[wave][2 * lane] = (u32x2) { 0u, 0u };
+    // MUL1: packed pairs against plain (x, x + 1) pairs: 4 MFMAs and 2 operand reads per slice, half
+    // the other codebooks' (lo, hi) against duplicated pairs
+    constexpr bool PAIRS = CB == 2;
+    constexpr int XW = PAIRS ? 8 : 16;                  // u32 per slice of staged x
     const bool diag = (lane & 15) == (lane >> 4);
     f32x4 accv[4] = { { 0, 0, 0, 0 }, { 0, 0, 0, 0 }, { 0, 0, 0, 0 }, { 0, 0, 0, 0 } };
     for (int c = 0; c < nchunks; ++c)
@@ -901,9 +949,10 @@ void gemv1_kernel(const GemvArgs g)
             const f16x2 p = as_h2(xr);
             const f16x2 d0 = { p.x, p.x }, d1 = { p.y, p.y };
             const int t = (2 * lane) & 15;
-            *(u32x2*) (xd + ((2 * lane) & ~15) + 4 * ((t & 7) >> 1) + 2 * (t >> 3)) = (u32x2) { as_u32(d0), as_u32(d1) };
+            if constexpr (PAIRS) xd[(lane >> 3) * 8 + 2 * ((t & 7) >> 1) + (t >> 3)] = xr;
+            else *(u32x2*) (xd + ((2 * lane) & ~15) + 4 * ((t & 7) >> 1) + 2 * (t >> 3)) = (u32x2) { as_u32(d0), as_u32(d1) };
         }
-        const uint32_t* bbase = diag ? xd + (lane0 / 8) * 16 : xzero[wave];
+        const uint32_t* bbase = diag ? xd + (lane0 / 8) * XW : xzero[wave];
         __builtin_amdgcn_wave_barrier();
         // prefetch the next chunk's x (clamped: stays inside this wave's range)
         const int cn = min(c + 1, nchunks - 1);
@@ -923,6 +972,25 @@ void gemv1_kernel(const GemvArgs g)
             // wait for the partial stores does not wait on HBM).  Unconditional, so the wait
             // counts stay static.
             load_slot_k<K>(i + PF <= last ? base + (size_t) (i + PF) * rstride : sinkp, prev_off, lane, ring[d]);
+            if constexpr (PAIRS)
+            {
+                uint32_t pk[16];
+                mul1_pairs<K>(wv, pk);
+                #pragma unroll
+                for (int gq = 0; gq < 2; ++gq)
+                {
+                    const f16x8 bx = __builtin_bit_cast(f16x8, *(const u32x4*) (bbase + s8 * XW + 4 * gq));
+                    #pragma unroll
+                    for (int cc = 0; cc < 2; ++cc)
+                    {
+                        const int q = 8 * gq + 2 * cc;
+                        const u32x4 aw = { pk[q], pk[q + 1], pk[q + 4], pk[q + 5] };
+                        accv[2 * gq + cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            __builtin_bit_cast(f16x8, aw), bx, accv[2 * gq + cc], 0, 0, 0);
+                    }
+                }
+            }
+            else
             // decode per group of 8 windows, right before its 2 MFMAs: 8 live words instead of 32
             #pragma unroll
             for (int gq = 0; gq < 4; ++gq)
@@ -997,7 +1065,7 @@ void gemv1_kernel(const GemvArgs g)
         res[c] = vv;
     }
     __syncthreads();
-    block_epilogue(g, v, j, chunk, slot, splits, res, tmp, &flag, svp);
+    block_epilogue<false>(g, v, j, chunk, slot, splits, res, tmp, &flag, svp);
     GEMV_STAMP(g, 3, flag);
 }
 
@@ -1244,9 +1312,14 @@ void gemv1b_kernel(const GemvArgs g)
 // column j + 8 c), B = the input at those rows of the lane's k-tile, read as one 16-byte LDS
 // load from the input staged in that row order (xperm).
 //
-// Workgroup: one 128-column chunk (4 waves = 4 column pairs) over SB k-tiles (SB % 8 == 0, so
-// the input rotation covers whole 128-row chunks); split-k partials and their hand-off are the
-// LDS kernel's (block_epilogue).
+// MUL1 weights are one fp16 each (1024 + byte sum) and come packed in pairs, so their A operands
+// hold 8 weights instead of 4 and the input is staged plain: 4 MFMAs and 2 operand reads per unit
+// instead of 8 and 4 (17408 -> 5120 at 2 bits, 8 rows: 28.8 -> 23.1 us with the staging below).
+//
+// Workgroup: one 128-column chunk (4 waves = 4 column pairs) over one of g.slots ranges of k, whole
+// 128-row chunks of the input, of equal length or one chunk more; slices_per_block is the
+// longest range's k-tiles (the LDS layout).  Split-k partials and their hand-off are the LDS
+// kernel's (block_epilogue).
 // ---------------------------------------------------------------------------------------------
 typedef _Float16 f16x8v __attribute__((ext_vector_type(8)));
 
@@ -1264,15 +1337,16 @@ void gemvm_kernel(const GemvArgs g)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t a3 = sconst(89226354u), b3 = vconst(64248484u);       // 3INST multiplier, addend
     const int m = g.m, k = g.k;
-    const int KS = k / 16;
-    const int SB = g.slices_per_block;                    // k-tiles per workgroup, multiple of 8
-    const int splits = KS / SB;
+    const int splits = g.slots;
     const int j = blockIdx.y;
     int chunk, slot;
     block_coords(g, splits, chunk, slot);
     MatView v;
     if (!resolve(g, j, v)) { inactive_arrive(g, chunk, slot, &flag); return; }
     if (chunk * 128 >= v.n) return;
+    // this slot's 128-row chunks of k: ranges of equal length, or one chunk more
+    const int kc0 = (int) ((long) (k / 128) * slot / splits), kc1 = (int) ((long) (k / 128) * (slot + 1) / splits);
+    const int SB = 8 * (kc1 - kc0), ks0 = 8 * kc0;        // k-tiles, first k-tile
     // the wave's start (staging) and end (hand-off) outrank the decode loops of the SIMD's other
     // waves, as in the M = 1 kernel
     __builtin_amdgcn_s_setprio(EXL3_GEMV_PRIO);
@@ -1285,54 +1359,79 @@ void gemvm_kernel(const GemvArgs g)
             g.trace[(((size_t) blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6)) * 8 + 5] = ((uint64_t) xcc << 32) | hw;
     }
 #endif
-    const int ks0 = slot * SB;
-    const int xs_stride = SB * 16 + 4;                    // u32 per row; +4: rows 16 bytes apart in the banks
-    uint32_t* xs = smem;                                  // [MT][xs_stride] dup pairs, xperm order
+    // MUL1 weights decode to packed pairs, so the rows are staged as they are; the other codebooks'
+    // (lo, hi) words meet duplicated (x, x) pairs
+    constexpr bool PAIRS = CB == 2;
+    constexpr int XW = PAIRS ? 8 : 16;                    // u32 per staged row and 16-row k-tile
+    const int xs_stride = g.slices_per_block * XW + 4;    // u32 per row; +4: rows 16 bytes apart in the banks
+    uint32_t* xs = smem;                                  // [MT][xs_stride], xperm order
     constexpr int RS = 132;                               // res row stride: 16-byte column groups of 16 rows in distinct banks
     float* res = (float*) (smem + MT * xs_stride);        // [MT][RS]
     float* tmp = res + MT * RS;                           // epilogue scratch: 2 x (m x 64 column pairs), >= 512
 
-    // Input rotation of the workgroup's SB / 8 chunks, every row, into xs (dup pairs, xperm order).
-    // Job q of wave w: row / chunk (w + 4 q) of m x SB / 8.  The first XB jobs' input and suh loads
-    // are issued before the weight ring's: loads return in issue order, so behind the ring they
-    // would wait for its HBM traffic.
-    constexpr int XB = 4;                                 // measured best of 2 / 4 / 8 / 16 (m = 2..8)
+    // Input rotation of the workgroup's nkc 128-row chunks, every row, into xs (xperm order): 16 lanes
+    // per (row, chunk) job as had128_kernel, lane g of a job holds rows 8 g .. 8 g + 7, so that a wave
+    // rotates 4 jobs in one chain of stages (one job per wave and chain, lane = two rows, took 7.1 us
+    // of a 25 us call at 8 rows of 5120 -> 17408).  The first XB steps' input and suh loads are
+    // issued before the weight ring's: loads return in issue order, so behind the ring they would
+    // wait for its HBM traffic.
+    constexpr int XB = 2;
     const int nkc = SB / 8, njobs = m * nkc;
-    uint32_t xr[XB], sr[XB];
+    const int jl = 4 * wave + (lane >> 4), jg = lane & 15;    // the lane's job of a step, its place in the job
+    u32x4 xr[XB], sr[XB];
     auto xload = [&](int jb) {
         #pragma unroll
         for (int q = 0; q < XB; ++q)
         {
-            const int job = min(jb + q * GEMV_WAVES, njobs - 1);
-            const int row = job / nkc, c = job % nkc;
-            const int col = ks0 * 16 + c * 128 + 2 * lane;
-            xr[q] = *to_global((const uint32_t*) (v.A + (size_t) row * k + col));
-            sr[q] = *to_global((const uint32_t*) ((v.suh ? v.suh : v.A) + col));   // unused without suh
+            const int job = min(jb + 16 * q + jl, njobs - 1);
+            const int row = job / nkc, c = job - row * nkc;
+            const int col = ks0 * 16 + c * 128 + 8 * jg;
+            xr[q] = *to_global((const u32x4*) (v.A + (size_t) row * k + col));
+            sr[q] = *to_global((const u32x4*) ((v.suh ? v.suh : v.A) + col));      // unused without suh
         }
     };
     auto xstage = [&](int jb) {
         #pragma unroll
         for (int q = 0; q < XB; ++q)
         {
-            const int job = jb + q * GEMV_WAVES;
-            if (job >= njobs) break;
-            const int row = job / nkc, c = job % nkc;
-            f16x2 o = as_h2(xr[q]);
+            const int job = jb + 16 * q + jl;
+            if (jb + 16 * q >= njobs) break;
+            const int row = job / nkc, c = job - row * nkc;
+            uint32_t xw[4] = { xr[q].x, xr[q].y, xr[q].z, xr[q].w };
             if (v.suh)
             {
-                const f16x2 xv = o * as_h2(sr[q]);
-                float v0 = (float) xv.x, v1 = (float) xv.y;
-                fwht128_wave(v0, v1, lane);
-                o.x = (f16) (v0 * EXL3_HAD_RSCALE);
-                o.y = (f16) (v1 * EXL3_HAD_RSCALE);
+                const uint32_t sw[4] = { sr[q].x, sr[q].y, sr[q].z, sr[q].w };
+                float e[8];
+                #pragma unroll
+                for (int i = 0; i < 4; ++i)
+                {
+                    const f16x2 xv = as_h2(xw[i]) * as_h2(sw[i]);
+                    e[2 * i] = (float) xv.x;
+                    e[2 * i + 1] = (float) xv.y;
+                }
+                fwht128_lane8(e, lane);
+                #pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    xw[i] = as_u32((f16x2) { (f16) (e[2 * i] * EXL3_HAD_RSCALE), (f16) (e[2 * i + 1] * EXL3_HAD_RSCALE) });
             }
-            const int e = 2 * lane;                       // even row of its 16-group: xperm(e+1) = xperm(e) + 1
-            const int pos = c * 128 + (e & ~15) + xperm(e & 15);
-            f16x2 d0 = { o.x, o.x }, d1 = { o.y, o.y };
-            *(u32x2*) (xs + row * xs_stride + pos) = (u32x2) { as_u32(d0), as_u32(d1) };
+            if (job >= njobs) continue;
+            // rows 8 g .. 8 g + 7 are one half h = g % 2 of 16-row k-tile g / 2: pair i goes to pair slot 2 i + h
+            uint32_t* xd = xs + row * xs_stride + (c * 8 + (jg >> 1)) * XW;
+            const int h = jg & 1;
+            #pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                if constexpr (PAIRS) xd[2 * i + h] = xw[i];
+                else
+                {
+                    const f16x2 o = as_h2(xw[i]);
+                    const f16x2 d0 = { o.x, o.x }, d1 = { o.y, o.y };
+                    *(u32x2*) (xd + 2 * (2 * i + h)) = (u32x2) { as_u32(d0), as_u32(d1) };
+                }
+            }
         }
     };
-    xload(wave);
+    xload(0);
     __builtin_amdgcn_sched_barrier(0);
 
     // this lane's tile: k-tile ks0 + lane / 16 (+ 4 per unit), column tile 2 wave + lane % 16 / 8
@@ -1351,8 +1450,8 @@ void gemvm_kernel(const GemvArgs g)
     // svh pair for the epilogue, behind the first weights
     const uint32_t svp = *to_global((const uint32_t*) ((v.svh ? v.svh + chunk * 128 : v.A) + 2 * lane));
 
-    xstage(wave);
-    for (int jb = wave + GEMV_WAVES * XB; jb < njobs; jb += GEMV_WAVES * XB)
+    xstage(0);
+    for (int jb = 16 * XB; jb < njobs; jb += 16 * XB)
     {
         xload(jb);
         xstage(jb);
@@ -1362,7 +1461,7 @@ void gemvm_kernel(const GemvArgs g)
     __builtin_amdgcn_s_setprio(0);
 
     const int nrow = min(lane & 15, m - 1);               // B column = activation row (clamped)
-    const uint32_t* xb = xs + nrow * xs_stride + (lane >> 4) * 16;
+    const uint32_t* xb = xs + nrow * xs_stride + (lane >> 4) * XW;
     f32x4 acc[2] = { { 0, 0, 0, 0 }, { 0, 0, 0, 0 } };
     for (int u0 = 0; u0 < nunits; u0 += PF)
     {
@@ -1374,19 +1473,39 @@ void gemvm_kernel(const GemvArgs g)
             uint32_t wv[KB + 1];
             #pragma unroll
             for (int w = 0; w <= KB; ++w) wv[w] = ring[d][w];
-            uint32_t raw[32];
-            raw32<K, CB>(wv, raw, a3, b3);
-            load_tile_lane<K>(tile0 + (size_t) min(u + PF, nunits - 1) * ustride, jt, prev_off, ring[d]);
-            #pragma unroll
-            for (int gq = 0; gq < 4; ++gq)
+            if constexpr (PAIRS)
             {
-                const u32x4 bx = *(const u32x4*) (xb + u * 64 + 4 * gq);
-                const f16x8v b = __builtin_bit_cast(f16x8v, bx);
+                uint32_t pk[16];
+                mul1_pairs<K>(wv, pk);
+                load_tile_lane<K>(tile0 + (size_t) min(u + PF, nunits - 1) * ustride, jt, prev_off, ring[d]);
                 #pragma unroll
-                for (int c = 0; c < 2; ++c)
+                for (int gq = 0; gq < 2; ++gq)
                 {
-                    const u32x4 aw = { raw[8 * gq + 4 * c], raw[8 * gq + 4 * c + 1], raw[8 * gq + 4 * c + 2], raw[8 * gq + 4 * c + 3] };
-                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8v, aw), b, acc[c], 0, 0, 0);
+                    const f16x8v b = __builtin_bit_cast(f16x8v, *(const u32x4*) (xb + u * 32 + 4 * gq));
+                    #pragma unroll
+                    for (int c = 0; c < 2; ++c)
+                    {
+                        const u32x4 aw = { pk[8 * gq + 2 * c], pk[8 * gq + 2 * c + 1], pk[8 * gq + 2 * c + 4], pk[8 * gq + 2 * c + 5] };
+                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8v, aw), b, acc[c], 0, 0, 0);
+                    }
+                }
+            }
+            else
+            {
+                uint32_t raw[32];
+                raw32<K, CB>(wv, raw, a3, b3);
+                load_tile_lane<K>(tile0 + (size_t) min(u + PF, nunits - 1) * ustride, jt, prev_off, ring[d]);
+                #pragma unroll
+                for (int gq = 0; gq < 4; ++gq)
+                {
+                    const u32x4 bx = *(const u32x4*) (xb + u * 64 + 4 * gq);
+                    const f16x8v b = __builtin_bit_cast(f16x8v, bx);
+                    #pragma unroll
+                    for (int c = 0; c < 2; ++c)
+                    {
+                        const u32x4 aw = { raw[8 * gq + 4 * c], raw[8 * gq + 4 * c + 1], raw[8 * gq + 4 * c + 2], raw[8 * gq + 4 * c + 3] };
+                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8v, aw), b, acc[c], 0, 0, 0);
+                    }
                 }
             }
         }
@@ -1409,7 +1528,11 @@ void gemvm_kernel(const GemvArgs g)
         for (int r = wave; r < m; r += GEMV_WAVES)
         {
             float sv = 0.0f;
-            for (int e = lane; e < SB * 16; e += 64) sv += (float) as_h2(xs[r * xs_stride + e]).x;
+            for (int e = lane; e < SB * XW; e += 64)
+            {
+                const f16x2 p = as_h2(xs[r * xs_stride + e]);
+                sv += (float) p.x + (float) p.y;
+            }
             sv = wave_sum(sv, lane);
             if (lane == 0) sumx[r] = sv;
         }
@@ -1425,15 +1548,14 @@ void gemvm_kernel(const GemvArgs g)
         }
         __syncthreads();
     }
-    block_epilogue(g, v, j, chunk, slot, splits, res, tmp, &flag, svp, RS);
+    block_epilogue<true>(g, v, j, chunk, slot, splits, res, tmp, &flag, svp, RS);
     GEMV_STAMP(g, 3, flag);
 }
 
 template <typename KernelLaunch>
 int launch_common(const GemvArgs& g, hipStream_t s, KernelLaunch main)
 {
-    const int KS = g.k / 16;
-    const int splits = KS / g.slices_per_block;
+    const int splits = g.slots;
     const int chunks = g.n / 128;
     main(dim3(splits * chunks, g.bszm));
     if (!g.xcd)
@@ -1478,7 +1600,7 @@ int launch_gemv1(const GemvArgs& g, hipStream_t s)
 template <int K, int CB, int MT>
 int launch_gemvm_t(const GemvArgs& g, hipStream_t s)
 {
-    const size_t lds = ((size_t) MT * (g.slices_per_block * 16 + 4) + (size_t) MT * 132 + (MT * 128 > 512 ? MT * 128 : 512)) * 4;
+    const size_t lds = ((size_t) MT * (g.slices_per_block * (CB == 2 ? 8 : 16) + 4) + (size_t) MT * 132 + (MT * 128 > 512 ? MT * 128 : 512)) * 4;
     return launch_common(g, s, [&](dim3 grid) {
         hipLaunchKernelGGL((gemvm_kernel<K, CB, MT>), grid, dim3(GEMV_THREADS), lds, s, g);
     });

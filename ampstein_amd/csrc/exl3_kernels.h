@@ -129,8 +129,9 @@ struct GemvArgs
     // work split (host planner)
     int stream_m1;              // 1: M = 1 streaming kernel, 0: LDS kernel
     int mfma_rows;              // 1: row-batched matrix-core kernel (gemvm_kernel, m <= 16)
-    int slices_per_block;       // SB: k-slices (16 rows x 128 columns) per workgroup, divides k/16
-    int slots;                  // split partials per column chunk: k/16 / SB
+    int slices_per_block;       // SB: k-slices (16 rows x 128 columns) per workgroup, divides k/16 (matrix-core
+                                // rows: those of the longest of `slots` near-equal ranges)
+    int slots;                  // split partials per column chunk
     int xs_chunks;              // rotated 128-row input chunks held in LDS (LDS kernel)
     int xcd;                    // > 0: XCD-local hand-off through L2 counters (workgroups b and b + xcd on one XCD)
     const uint32_t* sink;       // workspace: 8 KiB never written, target of the stream's past-the-end prefetches
