@@ -353,6 +353,7 @@ int gemv_plan(int m, int k, int n, int bszm, int num_cus, GemvArgs& g, size_t pa
                 const int nk = (blocks + sp - 1) / sp;           // 128-row chunks of the longest range
                 if ((size_t) mt * (nk * 128 + 4) * 4 > (size_t) GEMVM_STAGED_X_BYTES) continue;
                 if ((size_t) sp * bszm * m * n * 4 > partial_bytes && sp > 1) break;
+                if (best && (long) bszm * chunks * sp > 8L * num_cus) break;     // only slower from here on
                 const long per = ((long) bszm * chunks * sp + num_cus - 1) / num_cus;     // workgroups of a CU
                 const double t = 2.0 + per * 0.5 * ((double) blocks / sp + nk) * (0.5 + 0.027 * m) * (per == 1 ? 1.65 : 1.0) + 0.5 * per
                          + (sp > 1 ? 1.5 + 0.02 * m * sp : 0.0);

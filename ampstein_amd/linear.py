@@ -31,6 +31,7 @@ from .weights import Weights
 RECON_ROWS = 512
 ENGINE_RECON_ROWS = 144   # models.uc:35
 RECON_MAX_N = 32768       # models.uc:36
+NATIVE_ROWS = 1 << 30     # wider layers take exl3_gemm at any row count
 
 
 class LinearError(ValueError):
@@ -63,6 +64,12 @@ class LinearEXL3:
         self.out_features = shape[1] * 16
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # the exl3_gemm route in one native call, outputs included; None: x is of another form or the
+        # call is refused, and the statement below takes or refuses it
+        y = ops._native().linear_call(x, self.trellis, self.suh, self.svh, self.bias, self.mcg, self.mul1,
+                                      RECON_ROWS if self.out_features <= RECON_MAX_N else NATIVE_ROWS)
+        if y is not None:
+            return y
         m = x.size(0)
         if m > RECON_ROWS and self.out_features <= RECON_MAX_N:
             out = ops.exl3_gemm_recon(x.contiguous(), self.trellis, self.suh, self.svh, self.K,

@@ -38,6 +38,19 @@ RECON_FUSED_ROWS = int(os.environ.get("AMP_RECON_FUSED_ROWS", "2048")) or (1 << 
 # 2048 rows, measured: +4 % with the copy at 8192 -> 28672, -4 % at 28672 -> 8192).
 RECON_FUSED_X_SLABS_MIN_N = 16384
 
+_calls = None
+
+
+def _native():
+    """The native launch path (adapter/exl3_amd_torch.cpp gemm_call, linear_call, mgemm_call): checks
+    and launches in one call, and declines what the Python statement of the operator must refuse."""
+    global _calls
+    if _calls is None:
+        from . import torch_adapter
+        _calls = torch_adapter.load()
+    return _calls
+
+
 def _ptr(t: Optional[Tensor]):
     return None if t is None else t.data_ptr()
 
@@ -318,6 +331,13 @@ def exl3_gemm(A: Tensor, B: Tensor, C: Tensor, suh: Optional[Tensor], A_had: Opt
     A (..., k) fp16, B trellis (k/16, n/16, 16K) int16, C (..., n) fp16 or fp32.
     Returns the kernel tag (90 = GEMV, 91 = MFMA GEMM).  force_num_sms is accepted for
     interface parity (the reference's cooperative-grid override) and has no effect."""
+    native = _native()
+    try:
+        rc = native.gemm_call(A, B, C, suh, A_had, svh, force_shape_idx, mcg, mul1)
+    except TypeError:              # an argument of another type: converted, or refused, below
+        rc = native.DECLINED
+    if rc != native.DECLINED:
+        return check(rc)
     _need(B.dim() == 3, "B must be 3-dimensional")
     _need(A.size(-1) == B.size(0) * 16, "A and B shapes are incompatible")
     _need(C.size(-1) == B.size(1) * 16, "C and B shapes are incompatible")
@@ -425,6 +445,19 @@ def mgemm(x: Tensor, B_ptrs: Tensor, C: Tensor, suh_ptrs: Tensor, A_had: Tensor,
     C (num, m, n)) or, with opts {size_n_list, c_ptrs, n_stride_list, had_src_list,
     num_had_src}, sliced mode.  norm_in: see exl3_mgemm.  Returns C."""
     o = opts or {}
+    if norm_in is None:
+        native = _native()
+        rc = native.DECLINED
+        try:
+            if opts is None or (o.get("size_n_list") is not None and isinstance(o.get("num_had_src"), int)):
+                rc = native.mgemm_call(x, B_ptrs, C, suh_ptrs, A_had, svh_ptrs, K, mcg, mul1, o.get("size_n_list"),
+                                       o.get("c_ptrs"), o.get("n_stride_list"), o.get("had_src_list"),
+                                       o.get("num_had_src", 0))
+        except TypeError:          # an argument of another type: converted, or refused, below
+            pass
+        if rc != native.DECLINED:
+            check(rc)
+            return C
     if opts is not None:
         for key in ("size_n_list", "c_ptrs", "n_stride_list", "had_src_list"):
             _need(o.get(key) is not None, f"mgemm: opts.{key} missing")
