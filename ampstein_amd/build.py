@@ -46,6 +46,9 @@ def units():
     ]
     for cb in range(3):
         u.append(("exl3_moe.hip", f"exl3_moe_cb{cb}.o", [f"-DEXL3_MOE_CB={cb}"]))
+    for cb in (1, 2):            # grouped MoE GEMM: mcg, mul1; 16-row groups of a tile
+        for r in (8, 6, 4, 2):
+            u.append(("exl3_moeg.hip", f"exl3_moeg_cb{cb}_r{r}.o", [f"-DEXL3_MOEG_CB={cb}", f"-DEXL3_MOEG_R={r}"]))
     for k in range(1, 9):
         u.append(("exl3_gemv.hip", f"exl3_gemv_k{k}.o", [f"-DEXL3_INST_K={k}"]))
         u.append(("exl3_gemm.hip", f"exl3_gemm_k{k}.o", [f"-DEXL3_INST_K={k}"]))

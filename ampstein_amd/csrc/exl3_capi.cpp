@@ -1483,8 +1483,6 @@ int exl3_amd_moe(const uint16_t* hidden_state, int bsz, int hidden_dim, float* o
         const int v = policy(EXL3_AMD_POLICY_MOE_TILE_ROWS);
         if (reg_gemm ? (v == 32 || v == 64 || v == 96 || v == 128) : (v == 64 || v == 128 || v == 256)) tile_rows = v;
     }
-    // persistent moeg workgroups: 4 per CU
-    const int grid_wgs = d->num_cus * 4;
     const int rt_cap = pool / tile_rows + std::min(num_experts, pool) + 1;
     const size_t ps_floats = (size_t) pool * (2 * (hidden_dim / 128) + intermediate_dim / 128);
     // token-major output lists (atomic mode): starts, positions, build space, position -> row
@@ -1535,14 +1533,45 @@ int exl3_amd_moe(const uint16_t* hidden_state, int bsz, int hidden_dim, float* o
         exl3k_gemm_group_k1, exl3k_gemm_group_k2, exl3k_gemm_group_k3, exl3k_gemm_group_k4, exl3k_gemm_group_k5,
         exl3k_gemm_group_k6, exl3k_gemm_group_k7, exl3k_gemm_group_k8, exl3k_gemm_group_k17, exl3k_gemm_group_k18,
         exl3k_gemm_group_k19 };
-    static const group_fn gfn_reg[MOES_RATES] = {
-        exl3k_moeg_k1, exl3k_moeg_k2, exl3k_moeg_k3, exl3k_moeg_k4, exl3k_moeg_k5, exl3k_moeg_k6, exl3k_moeg_k7,
-        exl3k_moeg_k8, exl3k_moeg_k17, exl3k_moeg_k18, exl3k_moeg_k19 };
-    const group_fn* gfn = reg_gemm ? gfn_reg : gfn_lds;
+    typedef int (*moeg_fn)(const MoegArgs&, int, hipStream_t);
+    static const moeg_fn moeg[2][4] = {
+        { exl3k_moeg_cb1_r2, exl3k_moeg_cb1_r4, exl3k_moeg_cb1_r6, exl3k_moeg_cb1_r8 },
+        { exl3k_moeg_cb2_r2, exl3k_moeg_cb2_r4, exl3k_moeg_cb2_r6, exl3k_moeg_cb2_r8 } };
     const int cb = gate_mul1 ? 2 : 1;
     hipStream_t s = (hipStream_t) stream;
-    // one grouped launch per (phase, bitrate) that can occur: the list counts sit on the device
+    const int cus = d->num_cus;
+    // moeg: one launch per phase, which finds each list's bitrate on the device
+    auto moeg_phase = [&](int phase) -> int {
+        MoegArgs g;
+        memset(&g, 0, sizeof(g));
+        g.rt = a.rt;
+        g.nrt = rt_cap;
+        g.list_stride = rt_cap;
+        g.slots = bits_g ? 8 : MOES_RATES;                   // the tables hold integer widths
+        auto add = [&](int m, const uint16_t* A, uint16_t* C, const uint64_t* tab, const float* ps) {
+            g.A[g.mats] = A; g.C[g.mats] = C; g.tab[g.mats] = tab; g.psum[g.mats] = ps;
+            g.list[g.mats] = a.lists + (size_t) m * MOES_RATES * rt_cap;
+            g.count[g.mats] = a.counts + m * MOES_RATES;
+            ++g.mats;
+        };
+        if (phase == 0)
+        {
+            if (a.gated) add(0, a.ts_g, a.ti_g, a.g_trellis, a.ps_g);
+            add(1, a.ts_u, a.ti_u, a.u_trellis, a.ps_u);
+            g.k = hidden_dim; g.n = intermediate_dim;
+        }
+        else
+        {
+            add(2, a.ti_g, a.ts_g, a.d_trellis, a.ps_d);
+            g.k = intermediate_dim; g.n = hidden_dim;
+        }
+        // half rates have no mcg instance
+        if (cb == 1 && !bits_g && (phase ? a.K_d > 8 : a.K_u > 8 || (a.gated && a.K_g > 8))) return -1;
+        return moeg[cb - 1][tile_rows / 32 - 1](g, cus, s);
+    };
+    // LDS kernel: one grouped launch per (phase, bitrate) that can occur
     auto gemm_phase = [&](int phase) -> int {
+        if (reg_gemm) return moeg_phase(phase);
         for (int slot = 0; slot < MOES_RATES; ++slot)
         {
             const int K = moes_slot_rate(slot);
@@ -1551,33 +1580,31 @@ int exl3_amd_moe(const uint16_t* hidden_state, int bsz, int hidden_dim, float* o
             g.rt = a.rt;
             g.nrt = rt_cap;
             g.tile_rows = tile_rows;
-            g.grid_wgs = grid_wgs;
             int mats = 0;
-            auto add = [&](int m, const uint16_t* A, uint16_t* C, const uint64_t* tab, int Km, const float* ps) {
+            auto add = [&](int m, const uint16_t* A, uint16_t* C, const uint64_t* tab, int Km) {
                 if (bits_g ? K > 8 : Km != K) return;          // the tables hold integer widths
-                g.A[mats] = A; g.C[mats] = C; g.tab[mats] = tab; g.psum[mats] = ps;
+                g.A[mats] = A; g.C[mats] = C; g.tab[mats] = tab;
                 g.list[mats] = a.lists + (size_t) (m * MOES_RATES + slot) * rt_cap;
                 g.count[mats] = a.counts + m * MOES_RATES + slot;
                 ++mats;
             };
             if (phase == 0)
             {
-                if (a.gated) add(0, a.ts_g, a.ti_g, a.g_trellis, a.K_g, a.ps_g);
-                add(1, a.ts_u, a.ti_u, a.u_trellis, a.K_u, a.ps_u);
+                if (a.gated) add(0, a.ts_g, a.ti_g, a.g_trellis, a.K_g);
+                add(1, a.ts_u, a.ti_u, a.u_trellis, a.K_u);
                 g.k = hidden_dim; g.n = intermediate_dim;
             }
             else
             {
-                add(2, a.ti_g, a.ts_g, a.d_trellis, a.K_d, a.ps_d);
+                add(2, a.ti_g, a.ts_g, a.d_trellis, a.K_d);
                 g.k = intermediate_dim; g.n = hidden_dim;
             }
             if (!mats) continue;
             g.mats = mats;
-            if (int rc = gfn[slot](g, cb, s)) return rc;
+            if (int rc = gfn_lds[slot](g, cb, s)) return rc;
         }
         return 0;
     };
-    const int cus = d->num_cus;
     if (a.tok_start)
         if (int rc = exl3k_moes_tokens(a, s)) return hip_fail(rc, "exl3_moe");
     for (int row0 = 0; row0 < num_assign; row0 += pool)

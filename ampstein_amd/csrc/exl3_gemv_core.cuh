@@ -2,6 +2,7 @@
 // (exl3_moe.hip): trellis word loads, window extraction at compile-time offsets, codebook words
 // for the v_dot2 against (x, x) pairs.  See exl3_gemv.hip for the lane mapping.
 #pragma once
+#include <type_traits>
 
 #include "exl3_common.cuh"
 
@@ -171,5 +172,40 @@ __device__ __forceinline__ void raw32(const uint32_t* wv, uint32_t* raw, const u
 template <int K, int CB, int I>
 __device__ __forceinline__ uint32_t raw_at(const uint32_t* wv) { return raw_weight<CB>(state16<K, I>(wv)); }
 
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    if constexpr (I < N)
+    {
+        f(std::integral_constant<int, I> {});
+        static_for<I + 1, N>(f);
+    }
+}
+
+// Four 3INST / MCG weights' masked words r[2 i], r[2 i + 1] -> fp16 pairs (lo + hi each, one
+// rounding).  SDWA reads both halves of a word in one add and writes the half wanted: two
+// instructions per pair against three (two v_perm, v_pk_add_f16).  A destination half must not be
+// read by the next instruction, hence the order, and the s_nop behind the last one.
+__device__ __forceinline__ void sum_pairs4(const uint32_t* r, uint32_t* pk)
+{
+#define EXL3_LO(o, i) "v_add_f16_sdwa %" #o ", %" #i ", %" #i " dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+#define EXL3_HI(o, i) "v_add_f16_sdwa %" #o ", %" #i ", %" #i " dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+    asm(EXL3_LO(0, 4) EXL3_LO(1, 6) EXL3_LO(2, 8) EXL3_LO(3, 10)
+        EXL3_HI(0, 5) EXL3_HI(1, 7) EXL3_HI(2, 9) EXL3_HI(3, 11)
+        "s_nop 0"
+        : "=&v"(pk[0]), "=&v"(pk[1]), "=&v"(pk[2]), "=&v"(pk[3])
+        : "v"(r[0]), "v"(r[1]), "v"(r[2]), "v"(r[3]), "v"(r[4]), "v"(r[5]), "v"(r[6]), "v"(r[7]));
+#undef EXL3_LO
+#undef EXL3_HI
+}
+
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
+#define EXL3_WAIT_VM_LGKM0(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4))
+
+// Fewest vector-memory instructions that load_tile_lane<K> compiles to (neighbouring words may
+// be loaded together): the row waits count on at least this many per unit.
+constexpr int tile_lane_loads(int K) { return khalf(K) ? 2 : (K + 3) / 4 + 1; }
 
 }  // namespace exl3

@@ -214,9 +214,7 @@ struct GemmGroupArgs
     int mats;                   // 1 or 2
     int k, n;
     int nrt;                    // row-tile capacity of the launch
-    int tile_rows;              // rows per tile: 64, 128 or 256 (moeg: 32, 64 or 128)
-    int grid_wgs;               // moeg: persistent workgroups (0: one per item)
-    const float* psum[2];       // moeg, mul1: (pool rows, k / 128) chunk sums of A, per matrix set
+    int tile_rows;              // rows per tile: 64, 128 or 256
 };
 
 int exl3k_gemm_group_k1(const GemmGroupArgs& g, int cb, hipStream_t s);
@@ -227,21 +225,37 @@ int exl3k_gemm_group_k5(const GemmGroupArgs& g, int cb, hipStream_t s);
 int exl3k_gemm_group_k6(const GemmGroupArgs& g, int cb, hipStream_t s);
 int exl3k_gemm_group_k7(const GemmGroupArgs& g, int cb, hipStream_t s);
 int exl3k_gemm_group_k8(const GemmGroupArgs& g, int cb, hipStream_t s);
-// Register-decode grouped GEMM (exl3_gemm.hip moeg_kernel), same arguments.
-int exl3k_moeg_k1(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k2(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k3(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k4(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k5(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k6(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k7(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k8(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k17(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k18(const GemmGroupArgs& g, int cb, hipStream_t s);
-int exl3k_moeg_k19(const GemmGroupArgs& g, int cb, hipStream_t s);
 int exl3k_gemm_group_k17(const GemmGroupArgs& g, int cb, hipStream_t s);
 int exl3k_gemm_group_k18(const GemmGroupArgs& g, int cb, hipStream_t s);
 int exl3k_gemm_group_k19(const GemmGroupArgs& g, int cb, hipStream_t s);
+
+// Register-decode grouped GEMM of the token-sorted MoE (exl3_moeg.hip): one launch runs the row
+// tiles of every bitrate, from the same lists.
+struct MoegArgs
+{
+    const uint16_t* A[2];       // (pool rows, k) fp16, per matrix set
+    uint16_t* C[2];             // (pool rows, n) fp16
+    const uint64_t* tab[2];     // trellis address per expert
+    const float* psum[2];       // mul1: (pool rows, k / 128) chunk sums of A
+    const int* rt;              // row tiles: (expert, first row, rows) triples
+    const int* list[2];         // row-tile ids: slot s's list starts list_stride * s entries in
+    const int* count[2];        // entries in each slot's list
+    int mats;                   // 1 or 2
+    int k, n;
+    int nrt;                    // row-tile capacity
+    int list_stride;
+    int slots;                  // rate slots that may be run (8 or MOES_RATES)
+};
+
+// cb: 1 mcg, 2 mul1; r: 16-row groups of a tile
+int exl3k_moeg_cb1_r2(const MoegArgs& g, int cus, hipStream_t s);
+int exl3k_moeg_cb1_r4(const MoegArgs& g, int cus, hipStream_t s);
+int exl3k_moeg_cb1_r6(const MoegArgs& g, int cus, hipStream_t s);
+int exl3k_moeg_cb1_r8(const MoegArgs& g, int cus, hipStream_t s);
+int exl3k_moeg_cb2_r2(const MoegArgs& g, int cus, hipStream_t s);
+int exl3k_moeg_cb2_r4(const MoegArgs& g, int cus, hipStream_t s);
+int exl3k_moeg_cb2_r6(const MoegArgs& g, int cus, hipStream_t s);
+int exl3k_moeg_cb2_r8(const MoegArgs& g, int cus, hipStream_t s);
 
 // Token-sorted MoE (exl3_moe_sorted.hip).  Pool rows are the caller's temp buffers; the plan
 // tables live in the library workspace.

@@ -9,7 +9,8 @@
 //            max_tokens_per_expert rows), row tiles of <= 64 / 128 / 256 rows of one expert, and per
 //            (matrix, bitrate) lists of row tiles;
 //   gather   pool row r <- had(x[token] o suh) for gate and up (had_hf_r_128_inner);
-//   GEMM     grouped MFMA GEMM (exl3_gemm.hip, GROUP instance) per bitrate, gate and up together;
+//   GEMM     grouped MFMA GEMM of all bitrates (exl3_moeg.hip; or exl3_gemm.hip's GROUP instance, one
+//            launch per bitrate), gate and up together;
 //   act      had(g) o svh_g, had(u) o svh_u, act, limit, g * u, o suh_d, had (had_hf_r_128_guad_inner);
 //   GEMM     down;
 //   out      had(d) * (w / sqrt(128)) o svh_d added atomically to the token's row, or stored in its
@@ -105,7 +106,7 @@ __device__ __forceinline__ void hmul4(uint32_t* w, const uint32_t* s)
 __device__ __forceinline__ u32x4 ld16(const uint16_t* p) { return *to_global((const u32x4*) p); }
 
 // Sum of the 16-lane group's 128 fp16 values (lane g holds 8), in a fixed order: the row-chunk
-// sums the mul1 GEMM needs for its affine map (exl3_gemm.hip moeg_kernel).
+// sums the mul1 GEMM needs for its affine map (exl3_moeg.hip).
 __device__ __forceinline__ float group_sum16(const uint32_t* w)
 {
     float v = 0.0f;

@@ -35,8 +35,6 @@
 // Split k: each range stores its fp32 partial rows; the last arrival of a chunk (XCD-local
 // hand-off, exl3_xcd.cuh) adds them in k order, four rows in flight per wave, rotates and stores.
 // Without the hand-off exl3k_rows_finish does the same in a second launch.
-#include <type_traits>
-
 #include "exl3_common.cuh"
 #include "exl3_gemv_core.cuh"
 #include "exl3_kernels.h"
@@ -51,16 +49,12 @@ using namespace exl3;
 namespace {
 
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 constexpr int ROWS_KW = 2;                     // k halves of a workgroup
 constexpr int ROWS_THREADS = 256 * ROWS_KW;
 constexpr int ROWS_XNB = 4, ROWS_XD = ROWS_XNB - 1;   // row buffers (units) per k half, units in flight
 constexpr int ROWS_PF = 2;                     // trellis units in flight per wave
 constexpr int ROWS_RS = 132;                   // fp32 row stride of the reduction buffer
-
-// s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
-#define ROWS_VM_LGKM0(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4))
 
 template <int R> struct RowsLds
 {
@@ -69,37 +63,6 @@ template <int R> struct RowsLds
     static constexpr int RED = (ROWS_KW - 1) * RT * ROWS_RS;
     static constexpr int TOTAL = X > RED ? X : RED;
 };
-
-// Fewest vector-memory instructions that load_tile_lane<K> compiles to (neighbouring words may
-// be loaded together): the row wait below counts on at least this many per unit.
-constexpr int tile_lane_loads(int K) { return khalf(K) ? 2 : (K + 3) / 4 + 1; }
-
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    if constexpr (I < N)
-    {
-        f(std::integral_constant<int, I> {});
-        static_for<I + 1, N>(f);
-    }
-}
-
-// Four 3INST / MCG weights' masked words r[2 i], r[2 i + 1] -> fp16 pairs (lo + hi each, one
-// rounding).  SDWA reads both halves of a word in one add and writes the half wanted: two
-// instructions per pair against three (two v_perm, v_pk_add_f16).  A destination half must not be
-// read by the next instruction, hence the order, and the s_nop behind the last one.
-__device__ __forceinline__ void sum_pairs4(const uint32_t* r, uint32_t* pk)
-{
-#define EXL3_LO(o, i) "v_add_f16_sdwa %" #o ", %" #i ", %" #i " dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-#define EXL3_HI(o, i) "v_add_f16_sdwa %" #o ", %" #i ", %" #i " dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-    asm(EXL3_LO(0, 4) EXL3_LO(1, 6) EXL3_LO(2, 8) EXL3_LO(3, 10)
-        EXL3_HI(0, 5) EXL3_HI(1, 7) EXL3_HI(2, 9) EXL3_HI(3, 11)
-        "s_nop 0"
-        : "=&v"(pk[0]), "=&v"(pk[1]), "=&v"(pk[2]), "=&v"(pk[3])
-        : "v"(r[0]), "v"(r[1]), "v"(r[2]), "v"(r[3]), "v"(r[4]), "v"(r[5]), "v"(r[6]), "v"(r[7]));
-#undef EXL3_LO
-#undef EXL3_HI
-}
 
 // The lane's 32 windows as 16 packed pairs, eight windows at a time (bounded registers).
 template <int K, int CB>
@@ -208,7 +171,7 @@ void rows_kernel(const RowsArgs g)
             // loads issued after unit u's rows are done (loads complete in issue order)
             constexpr int VN = (ROWS_XD - 1) * ND + ROWS_XD * tile_lane_loads(K);
             static_assert(ROWS_PF <= ROWS_XD, "the wait assumes a trellis load between any two units' row loads");
-            ROWS_VM_LGKM0(VN < 60 ? VN : 60);
+            EXL3_WAIT_VM_LGKM0(VN < 60 ? VN : 60);
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -239,7 +202,7 @@ void rows_kernel(const RowsArgs g)
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    ROWS_VM_LGKM0(0);                                     // the past-the-end row loads still write LDS
+    EXL3_WAIT_VM_LGKM0(0);                                     // the past-the-end row loads still write LDS
     __syncthreads();
 
     // the k halves meet in LDS: D[i][nn] of acc[c][r] (lane: i = 4 (lane / 16) + e, nn = lane % 16) is

@@ -1,5 +1,5 @@
 """Host model of the token-sorted MoE's index structures (exl3_amd_moe, ampstein_amd/csrc/
-exl3_moe_sorted.hip and the moeg_kernel walk in exl3_gemm.hip), with a shadow-memory check of
+exl3_moe_sorted.hip and the moeg_kernel walk in exl3_moeg.hip), with a shadow-memory check of
 every workspace and pool-buffer read.
 
 What the kernels compute per call and per pass of `pool` rows (exl3_moe.cu:137-418 semantics):
