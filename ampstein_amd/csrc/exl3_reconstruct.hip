@@ -180,50 +180,38 @@ void reconstruct_t_kernel(uint16_t* __restrict__ WT, const uint16_t* __restrict_
 // -------------------------------------------------------------------------- reconstruct_had
 // One 128x128 block per workgroup.  LDS holds the block as 128 rows x 64 dwords with the
 // dword index of (row R, column pair cp) swizzled to cp ^ (2 * ((R >> 2) & 31)): conflict-free
-// for the column pass (32 lanes, 4 rows each, one column pair) and 8-byte aligned for the row
-// pass (32 lanes, 4 columns each).
+// for the column pass (16 column pairs x 4 rows, 32 apart) and 8-byte aligned and conflict-free for
+// the row pass (rows 4 apart x 4 column ranges).
+//
+// VALU- and LDS-bound (the 2.5 bytes a weight read and written would take 115 us at 8192 x 28672, 4 bits).  A lane holds 32 values of its column pair or row, so that three of the five fp16 stages
+// stay in its registers and two are quad DPP; with 4 values a lane all five went through the LDS
+// crossbar: 216 -> 182 us at that size (whole 2048-row product 1007 -> 980).
 __device__ __forceinline__ int rh_dw(int R, int cp) { return R * 64 + (cp ^ (((R >> 2) & 31) << 1)); }
 
 
-// fp16 lane stages xor 1..16 within a 32-lane half: lower lane a + b, upper (-b) + a
-// (shuffle_had_h2x32, hadamard_inner.cuh:83-93).  The partner value moves by DPP / permlane
-// (exl3_common.cuh xor_partner), not through LDS.
+// fp16 stage between quad lanes xor M (1, 2): lower lane a + b, upper a - b, as one v_pk_fma_f16 with a
+// +-1 factor (exactly v + p or p - v, one rounding).
 template <int M>
-__device__ __forceinline__ f16x2 had_h2_stage(f16x2 v, int lane)
+__device__ __forceinline__ f16x2 had_h2_quad(f16x2 v, int lane)
 {
-    // one v_pk_fma_f16 with a +-1 factor: exactly v + p (lower lane) or p - v (upper), one rounding
-    // the partner through the LDS crossbar: this kernel is VALU-bound (measured 8 % faster than
-    // the DPP partner)
-    const f16x2 p = as_h2(__builtin_bit_cast(uint32_t, xor_partner_sw<M>(__builtin_bit_cast(float, as_u32(v)))));
+    const f16x2 p = as_h2(__builtin_bit_cast(uint32_t, xor_partner<M>(__builtin_bit_cast(float, as_u32(v)), lane)));
     const f16 sg = (lane & M) ? (f16) -1.0f : (f16) 1.0f;
     const f16x2 sg2 = { sg, sg };
     return __builtin_elementwise_fma(v, sg2, p);
 }
 
-// Stage-major over N independent values, so each DPP read has other values' work in front of it
-// instead of the read-after-write wait states of one chain.
-template <int N>
-__device__ __forceinline__ void had_h2x32_n(f16x2 (&v)[N], int lane)
+// fp16 stage between elements i and i + W of N, in place.
+template <int W, int N>
+__device__ __forceinline__ void had_h2_inlane(f16x2 (&v)[N])
 {
     #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = had_h2_stage<1>(v[i], lane);
-    #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = had_h2_stage<2>(v[i], lane);
-    #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = had_h2_stage<4>(v[i], lane);
-    #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = had_h2_stage<8>(v[i], lane);
-    #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = had_h2_stage<16>(v[i], lane);
-}
-
-__device__ __forceinline__ f16x2 had_h2x32(f16x2 v, int lane)
-{
-    v = had_h2_stage<1>(v, lane);
-    v = had_h2_stage<2>(v, lane);
-    v = had_h2_stage<4>(v, lane);
-    v = had_h2_stage<8>(v, lane);
-    return had_h2_stage<16>(v, lane);
+    for (int i = 0; i < N; ++i)
+    {
+        if (i & W) continue;
+        const f16x2 a = v[i], b = v[i + W];
+        v[i] = a + b;
+        v[i + W] = a - b;
+    }
 }
 
 // TR: write the block transposed, WT (n, k) row-major (the layout the recon route's dense GEMM
@@ -260,60 +248,88 @@ void reconstruct_had_kernel(uint16_t* __restrict__ W, const uint16_t* __restrict
     __syncthreads();
 
     const f16x2 rs2 = { (f16) 0.08838834764831845f, (f16) 0.08838834764831845f };
-    const int t = lane & 31, half = lane >> 5;
+    const int qd = lane & 3, q16 = lane >> 2;
 
-    // 2. column pass (reconstruct.cu:290-325): per column pair, rows 4t..4t+3 in lane t;
-    //    fp16 4-point stage, times rs, fp16 lane stages
-    for (int it = 0; it < 8; ++it)
+    // 2. column pass (reconstruct.cu:290-325): rows 32 qd .. + 31 of column pair 16 wave + q16 in a lane, so
+    //    that three of the five fp16 stages (strides 4 .. 64 rows) stay in the lane and the last two are
+    //    quad DPP; fp16 4-point stage, times rs, fp16 stages.  The swizzle spreads the wave's reads of a
+    //    row offset over all banks.
     {
-        const int cp = (wave * 8 + it) * 2 + half;
-        f16x2 v[4];
+        const int cp = 16 * wave + q16;
+        f16x2 v[32];
         #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = as_h2(blk[rh_dw(4 * t + i, cp)]);
-        f16x2 s0 = v[0] + v[1], d0 = v[0] - v[1];
-        f16x2 s1 = v[2] + v[3], d1 = v[2] - v[3];
-        v[0] = (s0 + s1) * rs2;
-        v[1] = (d0 + d1) * rs2;
-        v[2] = (s0 - s1) * rs2;
-        v[3] = (d0 - d1) * rs2;
-        had_h2x32_n<4>(v, lane);
+        for (int i = 0; i < 32; ++i) v[i] = as_h2(blk[rh_dw(32 * qd + i, cp)]);
         #pragma unroll
-        for (int i = 0; i < 4; ++i) blk[rh_dw(4 * t + i, cp)] = as_u32(v[i]);
+        for (int i = 0; i < 32; i += 4)
+        {
+            const f16x2 s0 = v[i] + v[i + 1], d0 = v[i] - v[i + 1];
+            const f16x2 s1 = v[i + 2] + v[i + 3], d1 = v[i + 2] - v[i + 3];
+            v[i] = (s0 + s1) * rs2;
+            v[i + 1] = (d0 + d1) * rs2;
+            v[i + 2] = (s0 - s1) * rs2;
+            v[i + 3] = (d0 - d1) * rs2;
+        }
+        had_h2_inlane<4>(v);
+        had_h2_inlane<8>(v);
+        had_h2_inlane<16>(v);
+        #pragma unroll
+        for (int i = 0; i < 32; ++i) v[i] = had_h2_quad<1>(v[i], lane);
+        #pragma unroll
+        for (int i = 0; i < 32; ++i) v[i] = had_h2_quad<2>(v[i], lane);
+        #pragma unroll
+        for (int i = 0; i < 32; ++i) blk[rh_dw(32 * qd + i, cp)] = as_u32(v[i]);
     }
     __syncthreads();
 
-    // 3. row pass fused with the store (reconstruct.cu:331-357): row R, columns 4t..4t+3 in
-    //    lane t; fp32 4-point stage, round, times rs in fp16, fp16 lane stages, * suh * svh
-    const uint32_t sv01 = ((const uint32_t*) svh)[nb * 64 + 2 * t];
-    const uint32_t sv23 = ((const uint32_t*) svh)[nb * 64 + 2 * t + 1];
-    for (int it = 0; it < 16; ++it)
+    // 3. row pass (reconstruct.cu:331-357): columns 32 qd .. + 31 of row 64 it + 4 q16 + wave in a lane (as
+    //    above; rows 4 apart, for the banks); fp32 4-point stage, round, times rs in fp16, fp16 stages,
+    //    * suh * svh, back in place
+    uint32_t sv[16];
+    #pragma unroll
+    for (int j = 0; j < 16; ++j) sv[j] = ((const uint32_t*) svh)[nb * 64 + 16 * qd + j];
+    #pragma unroll
+    for (int it = 0; it < 2; ++it)
     {
-        const int R = (wave * 16 + it) * 2 + half;
-        const int d = rh_dw(R, 2 * t);
-        f16x2 a = as_h2(blk[d]), b = as_h2(blk[d + 1]);
-        float v0 = (float) a.x, v1 = (float) a.y, v2 = (float) b.x, v3 = (float) b.y;
-        float s0 = v0 + v1, d0 = v0 - v1, s1 = v2 + v3, d1 = v2 - v3;
-        f16x2 h01 = { (f16) (s0 + s1), (f16) (d0 + d1) };
-        f16x2 h23 = { (f16) (s0 - s1), (f16) (d0 - d1) };
-        h01 = h01 * rs2;
-        h23 = h23 * rs2;
-        f16x2 hh[2] = { h01, h23 };
-        had_h2x32_n<2>(hh, lane);
-        h01 = hh[0];
-        h23 = hh[1];
+        const int R = 64 * it + 4 * q16 + wave;
+        f16x2 h[16];
+        #pragma unroll
+        for (int j = 0; j < 16; j += 2)
+        {
+            const u32x2 w = *(const u32x2*) &blk[rh_dw(R, 16 * qd + j)];
+            const f16x2 a = as_h2(w.x), b = as_h2(w.y);
+            float v0 = (float) a.x, v1 = (float) a.y, v2 = (float) b.x, v3 = (float) b.y;
+            float s0 = v0 + v1, d0 = v0 - v1, s1 = v2 + v3, d1 = v2 - v3;
+            f16x2 h01 = { (f16) (s0 + s1), (f16) (d0 + d1) };
+            f16x2 h23 = { (f16) (s0 - s1), (f16) (d0 - d1) };
+            h[j] = h01 * rs2;
+            h[j + 1] = h23 * rs2;
+        }
+        had_h2_inlane<2>(h);
+        had_h2_inlane<4>(h);
+        had_h2_inlane<8>(h);
+        #pragma unroll
+        for (int j = 0; j < 16; ++j) h[j] = had_h2_quad<1>(h[j], lane);
+        #pragma unroll
+        for (int j = 0; j < 16; ++j) h[j] = had_h2_quad<2>(h[j], lane);
         const f16 su = as_h(suh[kb * 128 + R]);
         const f16x2 su2 = { su, su };
-        h01 = (h01 * su2) * as_h2(sv01);
-        h23 = (h23 * su2) * as_h2(sv23);
-        if constexpr (TR)
+        #pragma unroll
+        for (int j = 0; j < 16; j += 2)
         {
-            blk[d] = as_u32(h01);                          // in place: this lane's own words
-            blk[d + 1] = as_u32(h23);
+            const f16x2 h01 = (h[j] * su2) * as_h2(sv[j]), h23 = (h[j + 1] * su2) * as_h2(sv[j + 1]);
+            *(u32x2*) &blk[rh_dw(R, 16 * qd + j)] = (u32x2) { as_u32(h01), as_u32(h23) };   // this lane's own words
         }
-        else
+    }
+    __syncthreads();
+    if constexpr (!TR)
+    {
+        // 4. store: a half wave per row
+        const int t = lane & 31, half = lane >> 5;
+        #pragma unroll 4
+        for (int it = 0; it < 16; ++it)
         {
-            u32x2 o = { as_u32(h01), as_u32(h23) };
-            *(u32x2*) (W + (size_t) (kb * 128 + R) * n + nb * 128 + 4 * t) = o;
+            const int R = (wave * 16 + it) * 2 + half;
+            *(u32x2*) (W + (size_t) (kb * 128 + R) * n + nb * 128 + 4 * t) = *(const u32x2*) &blk[rh_dw(R, 2 * t)];
         }
     }
     if constexpr (TR)
@@ -323,9 +339,6 @@ void reconstruct_had_kernel(uint16_t* __restrict__ W, const uint16_t* __restrict
         //    row sit side by side: the swizzle flips even bits only), repacked by v_perm into four
         //    16-byte runs of 8 k, one per column.  Thread t takes units t and t + 256 (g = unit % 16,
         //    so 16 consecutive lanes store one column's 128 k contiguously; with slabs, 4 x 64 bytes).
-        //    (The former store, one u32 of two 16-bit LDS reads per lane and column, took ~290 us
-        //    at 8192 x 28672 against ~215 us for the (k, n) form.)
-        __syncthreads();
         #pragma unroll
         for (int u = 0; u < 2; ++u)
         {
