@@ -1473,8 +1473,9 @@ int exl3_amd_moe(const uint16_t* hidden_state, int bsz, int hidden_dim, float* o
     const bool reg_gemm = policy(EXL3_AMD_POLICY_MOE_GEMM) != EXL3_AMD_MOE_GEMM_LDS;
     // moeg: the smallest tile holding ~1.5x the mean rows (the largest expert, for top-k routing
     // of random tokens).  Measured, 256 experts 4096 -> 2048 -> 4096, top-8: T = 512 (mean 16,
-    // max 27) best at 32; T = 2048 (mean 64, max 91) best at 96: 2.32 ms against 2.49 at 64 and
-    // 2.54 at 128 (fewer tiles read each expert's weights fewer times; 96 keeps 3 waves per SIMD)
+    // max 27) best at 32 or 64 (0.99 / 1.07 ms); T = 1024 (mean 32) at 64: 1.19 against 1.48 at 32 and
+    // 1.35 at 96; T = 2048 (mean 64, max 91) at 96: 1.66 against 2.01 at 64 and 2.03 at 128 (fewer
+    // tiles decode each expert's weights fewer times; 96 keeps 3 waves per SIMD)
     const int want = mean_rows * 3 / 2;
     int tile_rows = reg_gemm ? (want <= 32 ? 32 : (want <= 64 ? 64 : (want <= 96 ? 96 : 128)))
                              : (mean_rows <= 40 ? 64 : (mean_rows <= 96 ? 128 : 256));
