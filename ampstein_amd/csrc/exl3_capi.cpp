@@ -391,9 +391,16 @@ int gemv_plan(int m, int k, int n, int bszm, int num_cus, GemvArgs& g, size_t pa
         if (best < 0 || (long) bszm * chunks * (KS / best) > target) best = d;   // fewest blocks >= target
         if ((long) bszm * chunks * (KS / d) <= target) break;
     }
-    // at least 3 workgroups per CU with whole columns (a vocabulary head): no split, so no hand-off
-    // or finish kernel (4096 -> 128256 at 6 bits: 98 us against 107 in two ranges)
-    const bool whole = stream && (long) bszm * chunks >= 3L * num_cus && ok_sb(KS);
+    // A vocabulary head: no split, so no hand-off or finish kernel, when whole columns give every CU at
+    // least 3 workgroups and their last round over the CUs is at most a tenth short.  Measured
+    // unsplit / best split, us (256 CUs): 4096 -> 128256 (3.91 workgroups per CU) at 4 / 6 bits 70 / 72 and
+    // 109 / 117, 2560 -> 151936 (4.64) 56 / 58 and 84 / 87, 2048 -> 262144 (8) 69 / 75 and 114 / 118;
+    // but 4096 -> 102400 (3.12: a fourth round for 32 of them) 67 / 60 and 102 / 95, 2048 -> 100352
+    // (3.06) 36 / 33 and 53 / 49, 4096 -> 49152 (1.5) 37 / 31 and 54 / 48.  Only where every workgroup is
+    // known to have work: with an index list or per-matrix widths most may have none (64 slots of
+    // 7168 -> 2048 at 4 bits with 8 in use: 39 us unsplit, 23 split).
+    const long wgs = (long) bszm * chunks, rounds = (wgs + num_cus - 1) / num_cus;
+    const bool whole = stream && !g.indices && !g.size_n && wgs >= 3L * num_cus && 10 * rounds * num_cus <= 11 * wgs && ok_sb(KS);
     // M = 1 stream: 4 k-slices per wave below k = 8192, 16 from there: the best splits measured
     // on MI355X for the Llama-3-8B shapes in a captured sweep (4096 x 4096: 6.85 -> 6.45 us, the
     // sliced q/k/v bundle 9.1 -> 7.9 us against 8 per wave; 14336 x 4096 best at 16)
