@@ -113,9 +113,12 @@ int mgemm_call(const at::Tensor& A, const at::Tensor& B, const at::Tensor& C, co
 PYBIND11_MODULE(exl3_amd_torch, m)
 {
     m.attr("DECLINED") = DECLINED;
-    m.def("gemm_call", &gemm_call);
-    m.def("linear_call", &linear_call);
-    m.def("mgemm_call", &mgemm_call);
+    // without the GIL, as the ctypes calls they stand for: a call can wait (the first one on a device
+    // allocates and synchronises, a launch waits on a full queue) while other Python threads run
+    const auto nogil = py::call_guard<py::gil_scoped_release>();
+    m.def("gemm_call", &gemm_call, nogil);
+    m.def("linear_call", &linear_call, nogil);
+    m.def("mgemm_call", &mgemm_call, nogil);
     m.def("exl3_gemm", [](const at::Tensor& A, const at::Tensor& B, at::Tensor C, const OptT& suh, const OptT& A_had,
                           const OptT& svh, int force_shape_idx, bool mcg, bool mul1, int force_num_sms) {
         return exl3_gemm(A, B, C, suh, A_had, svh, force_shape_idx, mcg, mul1, force_num_sms);

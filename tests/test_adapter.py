@@ -67,6 +67,43 @@ def test_adapter_rejects_bad_arguments(ad):
                          None, None, None, None, None)
 
 
+@pytest.mark.parametrize("call", ["gemm_call", "linear_call", "mgemm_call"])
+def test_native_calls_release_the_gil(ad, call):
+    """Under a switch interval longer than the test another thread runs only when this one lets go of
+    the GIL: between the native calls alone (here each declines its CPU tensors)."""
+    import sys
+    import threading
+    import time
+    h = lambda *s: torch.zeros(s, dtype=torch.half)
+    B, L = torch.zeros((8, 8, 64), dtype=torch.int16), torch.zeros(2, dtype=torch.long)
+    args = {"gemm_call": (h(1, 128), B, h(1, 128), None, None, None, 0, False, False),
+            "linear_call": (h(1, 128), B, h(128), h(128), None, False, False, 512),
+            "mgemm_call": (h(1, 1, 128), L, h(2, 1, 128), L, None, L, 4.0, False, False, None, None, None, None, 0)}[call]
+    fn = getattr(ad, call)
+    assert fn(*args) in (None, ad.DECLINED)
+    ticks, stop = [0], []
+
+    def other():
+        while not stop:
+            ticks[0] += 1
+            time.sleep(0)                          # lets go of the GIL itself
+    t = threading.Thread(target=other, daemon=True)
+    t.start()
+    prev = sys.getswitchinterval()
+    try:
+        sys.setswitchinterval(1000.0)
+        time.sleep(0.05)                           # the other thread now waits at the new interval
+        first, end = ticks[0], time.monotonic() + 3
+        while ticks[0] == first and time.monotonic() < end:
+            fn(*args)
+        seen = ticks[0] - first
+    finally:
+        stop.append(1)
+        sys.setswitchinterval(prev)
+    t.join(10)
+    assert seen > 0
+
+
 def gpu():
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
