@@ -129,6 +129,16 @@ def adapter_path() -> str:
     return os.path.join(LIB_DIR, "exl3_amd_torch" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
+def adapter_stale() -> bool:
+    """True when the adapter module is missing or older than its sources or the C header."""
+    out = adapter_path()
+    if not os.path.exists(out):
+        return True
+    deps = [os.path.join(ADAPTER_DIR, f) for f in os.listdir(ADAPTER_DIR) if f.endswith((".cpp", ".h"))]
+    deps.append(os.path.join(ROOT, "include", "exl3_amd.h"))
+    return max(os.path.getmtime(d) for d in deps) > os.path.getmtime(out)
+
+
 def build_adapter(verbose: bool = False) -> str:
     """The at::Tensor adapter (adapter/exl3_amd_adapter.cpp) and its Python module: host-only
     C++ (no device code) built by the host compiler against torch's ROCm headers, linked to
@@ -162,11 +172,11 @@ def build_adapter(verbose: bool = False) -> str:
 def main(argv=None):
     ap = argparse.ArgumentParser()
     ap.add_argument("-j", type=int, default=None)
-    ap.add_argument("--incremental", action="store_true", help="recompile stale units only; keep the adapter")
+    ap.add_argument("--incremental", action="store_true", help="recompile stale units, and the adapter when stale, only")
     args = ap.parse_args(argv)
     t0 = time.time()
     path = build(args.j, verbose=True, incremental=args.incremental)
-    if not args.incremental or not os.path.exists(adapter_path()):
+    if not args.incremental or adapter_stale():
         build_adapter(verbose=True)
     build_probe(verbose=True)
     print(f"built {path} in {time.time() - t0:.1f}s")

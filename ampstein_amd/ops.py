@@ -18,6 +18,7 @@ from __future__ import annotations
 from typing import Optional
 
 import os
+import warnings
 
 import torch
 
@@ -41,13 +42,40 @@ RECON_FUSED_X_SLABS_MIN_N = 16384
 _calls = None
 
 
+class _NoCalls:
+    """Stands for the native launch path where its module is missing: every call is declined."""
+    DECLINED = -1000000
+
+    @staticmethod
+    def gemm_call(*args):
+        return _NoCalls.DECLINED
+
+    mgemm_call = gemm_call
+
+    @staticmethod
+    def linear_call(*args):
+        return None
+
+
 def _native():
     """The native launch path (adapter/exl3_amd_torch.cpp gemm_call, linear_call, mgemm_call): checks
-    and launches in one call, and declines what the Python statement of the operator must refuse."""
+    and launches in one call, and declines what the Python statement of the operator must refuse.
+    The operators need libexl3_amd.so alone: without the module, or with one built before it had
+    these calls, the Python statement makes the same library call (about 8 us more of host time)."""
     global _calls
     if _calls is None:
         from . import torch_adapter
-        _calls = torch_adapter.load()
+        try:
+            mod = torch_adapter.load()
+            missing = [n for n in ("DECLINED", "gemm_call", "linear_call", "mgemm_call") if not hasattr(mod, n)]
+            why = f"has no {missing[0]}" if missing else None
+        except ImportError as e:
+            mod, why = None, f"is not loadable ({e})"
+        if why:
+            warnings.warn(f"the exl3_amd_torch module {why}: the operators launch through ctypes, which takes longer "
+                          "per call (python -m ampstein_amd.build builds it)", RuntimeWarning, stacklevel=3)
+            mod = _NoCalls
+        _calls = mod
     return _calls
 
 

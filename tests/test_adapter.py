@@ -67,6 +67,44 @@ def test_adapter_rejects_bad_arguments(ad):
                          None, None, None, None, None)
 
 
+@pytest.mark.parametrize("form", ["missing", "older"])
+def test_operators_without_the_module(monkeypatch, form):
+    """No adapter module, or one without the native calls: a warning, and the Python statement of every
+    operator (here its refusal of CPU tensors)."""
+    from ampstein_amd import _lib, ops
+    from ampstein_amd.linear import LinearEXL3
+
+    def load():
+        if form == "missing":
+            raise ImportError("not built")
+        return type("older", (), {"exl3_gemm": None})
+    monkeypatch.setattr(ops, "_calls", None)
+    monkeypatch.setattr(torch_adapter, "load", load)
+    h = lambda *s: torch.zeros(s, dtype=torch.half)
+    B, L = torch.zeros((8, 8, 64), dtype=torch.int16), torch.zeros(2, dtype=torch.long)
+    with pytest.warns(RuntimeWarning, match="exl3_amd_torch"), pytest.raises(_lib.Exl3Error, match="GPU"):
+        ops.exl3_gemm(h(1, 128), B, h(1, 128), None, None, None)
+    with pytest.raises(_lib.Exl3Error, match="GPU"):
+        ops.mgemm(h(1, 1, 128), L, h(2, 1, 128), L, None, L, 4.0, False, False)
+    lin = LinearEXL3.__new__(LinearEXL3)
+    lin.trellis, lin.suh, lin.svh, lin.bias, lin.mcg, lin.mul1 = B, h(128), h(128), None, False, False
+    lin.in_features = lin.out_features = 128
+    with pytest.raises(_lib.Exl3Error, match="GPU"):
+        lin(h(1, 128))
+
+
+def test_incremental_build_sees_a_stale_module(monkeypatch, tmp_path):
+    import os
+    from ampstein_amd import build
+    so = tmp_path / "module.so"
+    monkeypatch.setattr(build, "adapter_path", lambda: str(so))
+    assert build.adapter_stale()
+    so.write_bytes(b"")
+    assert not build.adapter_stale()
+    os.utime(so, (1, 1))
+    assert build.adapter_stale()
+
+
 @pytest.mark.parametrize("call", ["gemm_call", "linear_call", "mgemm_call"])
 def test_native_calls_release_the_gil(ad, call):
     """Under a switch interval longer than the test another thread runs only when this one lets go of
