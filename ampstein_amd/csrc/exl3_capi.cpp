@@ -963,6 +963,10 @@ int exl3_amd_to_slabs(const uint16_t* x, uint16_t* y, int rows, int cols, int ro
 
 namespace {
 
+// The kernels that stage rows with global_load_lds_dwordx4 take them from 16-byte aligned addresses
+// only; plain loads take any.  Rows are multiples of 256 bytes, so the base decides.
+bool dma_aligned(const void* p) { return ((uintptr_t) p & 15) == 0; }
+
 // exl3_gemm on a given workspace (the library's per-device one, or the no-alloc scratch).
 // ws == nullptr: the library's, set up on first use.
 int gemm_impl(const Workspace* ws, const uint16_t* A, const uint16_t* trellis, void* C, int c_fp32,
@@ -1021,7 +1025,9 @@ int gemm_impl(const Workspace* ws, const uint16_t* A, const uint16_t* trellis, v
     // tile, as many as fill the CUs, at least 4 stages of 32 k each, the S fp32 partial tiles
     // within the workspace; the fixup kernel sums them in k order and runs the epilogue.
     const long blocks = (long) ((n + 255) / 256) * ((m + 255) / 256);
-    const int staging = policy(EXL3_AMD_POLICY_GEMM_STAGING);
+    // rows that the LDS DMA cannot take: the GEMV groups or the register-staged tiles
+    const bool aligned = dma_aligned(A_rot);
+    const int staging = aligned ? policy(EXL3_AMD_POLICY_GEMM_STAGING) : EXL3_AMD_GEMM_STAGING_REGS;
     int splits = 1;
     if (staging == 0 && 2 * blocks <= ws->num_cus)
     {
@@ -1035,7 +1041,7 @@ int gemm_impl(const Workspace* ws, const uint16_t* A, const uint16_t* trellis, v
     {
         const long rounds = (blocks + ws->num_cus - 1) / ws->num_cus;
         const double t_gemm = 22.0 + (splits > 1 ? 0.030 * k / splits + 1e-6 * splits * (double) m * n : 0.030 * k * rounds);
-        const double t_group = m <= 16 ? 8.0 + 3.7e-7 * (double) n * k : 1e30;
+        const double t_group = m <= 16 || !aligned ? ((m + 15) / 16) * (8.0 + 3.7e-7 * (double) n * k) : 1e30;
         RowsArgs rr;
         memset(&rr, 0, sizeof(rr));
         rr.A_rot = A_rot;
@@ -1477,7 +1483,9 @@ int exl3_amd_moe(const uint16_t* hidden_state, int bsz, int hidden_dim, float* o
     // GEMM kernel: the register-decode moeg_kernel (default) or the LDS-tiled gemm_kernel
     // (policy EXL3_AMD_POLICY_MOE_GEMM = EXL3_AMD_MOE_GEMM_LDS).  moeg rows per tile: one tile per
     // expert for most experts
-    const bool reg_gemm = policy(EXL3_AMD_POLICY_MOE_GEMM) != EXL3_AMD_MOE_GEMM_LDS;
+    // (the LDS-tiled one also where moeg's LDS DMA cannot take the caller's row buffers)
+    const bool reg_gemm = policy(EXL3_AMD_POLICY_MOE_GEMM) != EXL3_AMD_MOE_GEMM_LDS && dma_aligned(temp_state_g) &&
+                          dma_aligned(temp_state_u) && dma_aligned(temp_intermediate_g);
     // moeg: the smallest tile holding ~1.5x the mean rows (the largest expert, for top-k routing
     // of random tokens).  Measured, 256 experts 4096 -> 2048 -> 4096, top-8: T = 512 (mean 16,
     // max 27) best at 32 or 64 (0.99 / 1.07 ms); T = 1024 (mean 32) at 64: 1.19 against 1.48 at 32 and

@@ -64,7 +64,7 @@ def model(es, x, flat, token_sorted, weight_sorted, count, start, max_tok, lo, h
     return out, slot_rows
 
 
-def run_moe(es, x, rt, max_tok, concurrency, lo, hi, act, limit, Ks, scratch_mode=False, m_tile=16, poison=False):
+def run_moe(es, x, rt, max_tok, concurrency, lo, hi, act, limit, Ks, scratch_mode=False, m_tile=16, poison=False, offset=0):
     flat, order, inv, token_sorted, weight_sorted, count, start = rt
     from ampstein_amd import ops
     T, H = x.shape
@@ -72,8 +72,10 @@ def run_moe(es, x, rt, max_tok, concurrency, lo, hi, act, limit, Ks, scratch_mod
     dev = "cuda"
     xs = torch.from_numpy(x).to(dev)
     out = torch.zeros((T, H), dtype=torch.float, device=dev)
-    ts = [torch.zeros((concurrency, max_tok, H), dtype=torch.half, device=dev) for _ in range(2)]
-    ti = [torch.zeros((concurrency, max_tok, I), dtype=torch.half, device=dev) for _ in range(2)]
+    # (offset: elements between the allocation's start and the row buffers')
+    zeros = lambda w: torch.zeros(concurrency * max_tok * w + offset, dtype=torch.half, device=dev)[offset:].view(concurrency, max_tok, w)
+    ts = [zeros(H) for _ in range(2)]
+    ti = [zeros(I) for _ in range(2)]
     tb = es.tables
     mcg, mul1 = es.cb == 1, es.cb == 2
     bits = (None, None, None)
