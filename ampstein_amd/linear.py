@@ -75,8 +75,9 @@ class LinearEXL3:
             out = ops.exl3_gemm_recon(x.contiguous(), self.trellis, self.suh, self.svh, self.K,
                                       self.mul1, self.mcg)
         else:
-            if m > ENGINE_RECON_ROWS:
-                # the engine's recon range: its input checks, and x in any strides
+            if m > ENGINE_RECON_ROWS and self.out_features <= RECON_MAX_N:
+                # the engine's recon range: its input checks, and x in any strides.  (Wider layers take
+                # exl3_gemm there too, and what it takes: x of any rank, contiguous.)
                 ops._need(x.dim() == 2 and x.size(1) == self.in_features and self.suh.numel() == self.in_features
                           and self.svh.numel() == self.out_features,
                           f"LinearEXL3: incompatible shapes (x {tuple(x.shape)}, weight {self.in_features} x "

@@ -3,8 +3,8 @@
 CPU: a synthetic EXL3 checkpoint written with safetensors, single-file and sharded (index
 json), read back key by key; K / codebook / feature counts derived from the trellis shape and
 the marker tensors, and the reference's rejections (both markers, half K without mul1,
-unknown key).  GPU: forward() on both routes (decode GEMM at few rows, reconstruct + dense
-GEMM above 144 rows), with and without bias, against the CPU oracle's fp64 linear.
+unknown key).  GPU: forward() on both routes (exl3_gemm up to 512 rows, reconstruct + dense GEMM
+above), with and without bias, against the CPU oracle's fp64 linear.
 """
 import json
 import os
@@ -113,6 +113,31 @@ def test_linear_rejections(tmp_path):
         LinearEXL3(ws, "half")
     with pytest.raises(WeightsError):
         LinearEXL3(ws, "absent")
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("rows", [144, 145, 512])
+def test_linear_forms_past_the_engine_line(tmp_path, monkeypatch, rows, wide):
+    """Layers wider than the recon route's limit hand exl3_gemm x as it is at any row count (3-D rows taken,
+    other strides for exl3_gemm to refuse); narrower ones take the recon route's 2-D x in any strides
+    above 144 rows."""
+    from ampstein_amd import _lib, linear, ops
+    L = synth.layer(256, 384, 4, 0, seed=6)
+    _write_model(str(tmp_path), _layer_tensors("m.q", L), False)
+    lin = linear.LinearEXL3(_CpuWeights(open_weights(str(tmp_path))), "m.q")
+    monkeypatch.setattr(linear, "RECON_MAX_N", 256 if wide else 384)
+    seen = []
+    monkeypatch.setattr(ops, "exl3_gemm", lambda x, *a: seen.append(x))
+    x = torch.zeros((rows, 512), dtype=torch.half)[:, :256]
+    lin(x)
+    assert seen[-1].is_contiguous() == (rows > 144 and not wide)
+    x3 = torch.zeros((rows, 1, 256), dtype=torch.half)
+    if rows > 144 and not wide:
+        with pytest.raises(_lib.Exl3Error, match="incompatible shapes"):
+            lin(x3)
+    else:
+        lin(x3)
+        assert seen[-1] is x3
 
 
 @pytest.mark.gpu
