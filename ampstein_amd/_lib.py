@@ -149,6 +149,7 @@ POLICY_GEMV_SPLIT, GEMV_SPLIT_BALANCED = 6, 1
 POLICY_GEMV_SLICES = 7
 POLICY_XCD_FAKE = 8
 POLICY_MOE_EPILOGUE, MOE_EPILOGUE_SERIAL = 9, 1
+POLICY_GEMM_KERNEL, GEMM_KERNEL_ROWS = 10, 1
 
 
 class policy:

@@ -82,7 +82,10 @@ int exl3_amd_version(void);
                                                  instead of the forms that issue every load first
                                                  (gate/up: at most 4 k-splits; down: top-k <= 16, at
                                                  most 2 k-splits); same bits                            */
-#define EXL3_AMD_POLICY_COUNT           10
+#define EXL3_AMD_POLICY_GEMM_KERNEL     10  /* kernel of exl3_amd_gemm above 8 rows with force_shape_idx 0:
+                                             * 0 = by the time models                                  */
+#define EXL3_AMD_GEMM_KERNEL_ROWS       1   /*   the row tiles (exl3_rows.hip) wherever they can run    */
+#define EXL3_AMD_POLICY_COUNT           11
 int exl3_amd_set_policy(int key, int value);
 int exl3_amd_get_policy(int key);       /* the current value, or EXL3_AMD_EINVAL for an unknown key */
 

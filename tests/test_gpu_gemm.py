@@ -108,25 +108,36 @@ def test_gemm_shapes(torch_cuda, orc, m, k, n, y_fp32):
     assert np.array_equal(A_had.view(np.uint16), orc.had128(x, pre=L.suh).view(np.uint16))
 
 
-@pytest.mark.parametrize("m,k,n,K,cb,route", [(9, 5120, 17408, 2, 0, 90), (16, 17408, 5120, 4, 1, 90),
-                                                (33, 4096, 14336, 3, 2, 91), (64, 5120, 5120, 2.5, 2, 91),
-                                                (100, 4096, 1024, 4, 0, 91)])
-def test_gemm_medium_batch_routing(torch_cuda, orc, m, k, n, K, cb, route):
-    """m > 8 with few 256-row tiles per CU: one or two 16-row groups of the matrix-core GEMV (tag
-    90) against the MFMA GEMM with its k split (tag 91, from ~32 rows), by the library's time
-    model; the rotated input written into A_had either way; the call forced onto the MFMA GEMM
-    agrees."""
+@pytest.mark.parametrize("m,k,n,K,cb,route", [(9, 5120, 17408, 2, 0, "rows"), (16, 17408, 5120, 4, 1, "rows"),
+                                                (33, 4096, 14336, 3, 2, "rows"), (64, 5120, 5120, 2.5, 2, "rows"),
+                                                (100, 4096, 1024, 4, 0, "tiled"), (12, 1024, 4096, 4, 0, "gemv"),
+                                                (16, 4096, 1024, 3, 2, "gemv"), (300, 4096, 1024, 3, 1, "rows")])
+def test_gemm_medium_batch_routing(torch_cuda, orc, kernel_policy, m, k, n, K, cb, route):
+    """m > 8 with few 256-row tiles per CU: the matrix-core GEMV (up to 16 rows, tag 90), the row tiles (tag 90
+    up to 16 rows, else 91) or the tiled GEMM with its k split (tag 91), by the library's time models (for
+    256 CUs).  Which one ran shows in the bits: each adds its fp32 sums in an order of its own.  The
+    rotated input is written into A_had on every route."""
     torch = torch_cuda
     L = synth.layer(k, n, K, cb, seed=650 + m + n)
     x = synth.activations(m, k, seed=651 + m)
-    tag, y, A_had = run_gemm(torch, L, x, False, force=0)
-    assert tag == route
+    tag, y16, A_had = run_gemm(torch, L, x, False, force=0)
+    assert tag == (90 if m <= 16 else 91)
     assert np.array_equal(A_had.view(np.uint16), orc.had128(x, pre=L.suh).view(np.uint16))
     ref = orc.linear_f64(x, L.trellis, L.suh, L.svh, int(K), half=K != int(K), cb=cb)
-    assert rel_err(y, ref) < TOL
-    tag2, y2, _ = run_gemm(torch, L, x, False, force=2)
+    assert rel_err(y16, ref) < TOL
+    _, y, _ = run_gemm(torch, L, x, True, force=0)
+    forced = {}
+    if m <= 16:
+        tag1, forced["gemv"], _ = run_gemm(torch, L, x, True, force=1)
+        assert tag1 == 90
+    tag2, forced["tiled"], _ = run_gemm(torch, L, x, True, force=2)
     assert tag2 == 91
-    assert rel_err(y2, ref) < TOL
+    kernel_policy(_lib.POLICY_GEMM_KERNEL, _lib.GEMM_KERNEL_ROWS)
+    _, forced["rows"], _ = run_gemm(torch, L, x, True, force=0)
+    for r, yf in forced.items():
+        assert rel_err(yf, ref) < TOL
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert [r for r, yf in forced.items() if np.array_equal(y, yf)] == [route]
 
 
 @pytest.mark.parametrize("suh,svh", [(False, False), (True, False), (False, True)])
