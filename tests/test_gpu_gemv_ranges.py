@@ -20,12 +20,12 @@ def torch_cuda():
     return torch
 
 
-def gemm(torch, L, x):
+def gemm(torch, L, x, force=0):
     from ampstein_amd import ops
     t, s, v = L.torch()
     A = torch.from_numpy(x).cuda()
     C = torch.full((x.shape[0], L.n), float("nan"), dtype=torch.half, device="cuda")
-    call = lambda: ops.exl3_gemm(A, t, C, s, torch.empty_like(A), v, 0, L.cb == 1, L.cb == 2)
+    call = lambda: ops.exl3_gemm(A, t, C, s, torch.empty_like(A), v, force, L.cb == 1, L.cb == 2)
     assert call() == 90
     return C, call
 
@@ -46,10 +46,25 @@ def check(C, ref, what):
 @pytest.mark.parametrize("k,n", [(128, 1024), (896, 1024), (1408, 384), (5248, 1024)])
 @pytest.mark.parametrize("K,cb", [(4, 0), (3, 1), (5, 2), (2.5, 2)])
 def test_rows_ranges(torch_cuda, orc, m, k, n, K, cb):
-    """1, 7, 11 and 41 chunks of 128 rows: no divisor but one; odd numbers of (row, chunk) jobs."""
+    """1, 7, 11 and 41 chunks of 128 rows: no divisor but one; odd numbers of (row, chunk) jobs.  On 256 CUs
+    the planner takes 1, 7 and 11 ranges of one chunk each, and 21 or 22 unequal ones of 41 chunks."""
+    ranges(torch_cuda, orc, m, k, n, K, cb, 0)
+
+
+@pytest.mark.parametrize("m,k,n", [(m, 5248, n) for m in (3, 4, 8) for n in (384, 1152)]
+                         + [(m, k, n) for m in (9, 12, 16) for k, n in ((5248, 384), (5248, 1024), (1408, 384))])
+@pytest.mark.parametrize("K,cb", [(4, 0), (3, 1), (5, 2), (2.5, 2)])
+def test_rows_unequal_ranges(torch_cuda, orc, m, k, n, K, cb):
+    """Unequal ranges (256 CUs: 21 of 41 chunks at 3..8 rows; 14 of 41, and 6 of 11 at 16 rows, at 9..16
+    rows) with the finish kernel (n / 128 = 3, 9) and the hand-off; the 9..16-row instance, which exl3_gemm
+    takes under force_shape_idx 1 at any size."""
+    ranges(torch_cuda, orc, m, k, n, K, cb, 1)
+
+
+def ranges(torch_cuda, orc, m, k, n, K, cb, force):
     L = synth.layer(k, n, K, cb, seed=9000 + k + m + int(10 * K))
     x = synth.activations(m, k, seed=9001 + k)
-    C, call = gemm(torch_cuda, L, x)
+    C, call = gemm(torch_cuda, L, x, force)
     check(C, orc.linear_f64(x, L.trellis, L.suh, L.svh, int(K), half=K != int(K), cb=cb), (m, k, n, K, cb))
     first = C.clone()
     call()
