@@ -133,6 +133,33 @@ def plan(count, E, num_assign, max_tok, lo, hi, pool, tile_rows, w0, Kcodes):
     return rowinfo, tiles, lists, inv, total
 
 
+def moeg_walk(counts, mats, nch, slots, grid):
+    """The item loop of moeg_kernel (exl3_moeg.hip): counts[i][slot] entries of matrix set i's list of each
+    rate slot, nch column chunks, `grid` workgroups (a multiple of 8).  Yields (workgroup, matrix set,
+    slot, index in the slot's list, chunk)."""
+    # ends[32 m + s]: entries of matrix set m in the lists of slots slots - 1 .. slots - 1 - s (the kernel's
+    # scan over 32 lanes, of which the first 16 are complete)
+    ends = np.zeros(64, np.int64)
+    for t in range(64):
+        m, s = t >> 5, t & 31
+        if m < mats and s < slots:
+            ends[t] = counts[m][slots - 1 - s]
+    for o in (1, 2, 4, 8):
+        ends = np.array([ends[t] + (ends[t - o] if (t & 31) >= o else 0) for t in range(64)])
+    tot = (int(ends[15]), int(ends[47]))
+    ents = max(tot) * mats
+    for wg in range(grid):
+        xcd, lb, nlb = wg & 7, wg >> 3, grid >> 3
+        per_xcd = (ents - xcd + 7) // 8 if ents > xcd else 0
+        for it in range(lb, per_xcd * nch, nlb):
+            ent, chunk = xcd + 8 * (it // nch), it % nch
+            m, pos = ent % mats, ent // mats
+            if pos >= tot[m]:
+                continue
+            s = int(np.count_nonzero(ends[32 * m:32 * m + 16] <= pos))
+            yield wg, m, slots - 1 - s, pos - (int(ends[32 * m + s - 1]) if s else 0), chunk
+
+
 class Shadow:
     """Per-element pass stamps of one buffer: -1 = not written in this call."""
 
@@ -149,9 +176,13 @@ class Shadow:
 
 
 def simulate(count, token_sorted, T, E, H, I, max_tok, conc, lo, hi, Kcodes, gated=True, tile_rows=None,
-             tok_mode=True):
+             tok_mode=True, slots=None, grid=1024):
     """Replay one exl3_amd_moe call's index walks; assert that every read hits memory written in
-    the same pass (or is rejected by its guard).  Returns per-token contributions per pass."""
+    the same pass (or is rejected by its guard).  slots: rate slots the grouped GEMM walks (8 with
+    per-expert rate tables, which hold integer widths, else 11); grid: its workgroups at most.
+    Returns per-token contributions per pass."""
+    if slots is None:
+        slots = 8 if all(int(c) <= 8 for codes in Kcodes for c in codes) else MOES_RATES
     num_assign = len(token_sorted)
     pool = min(conc * max_tok, num_assign)
     tr = tile_rows or tile_rows_for(num_assign, E)
@@ -202,21 +233,30 @@ def simulate(count, token_sorted, T, E, H, I, max_tok, conc, lo, hi, Kcodes, gat
             ps["u"].write(r, p)
 
         def gemm(phase):
-            mats = ([0] if gated else []) + [1] if phase == 0 else [2]
-            for s in range(MOES_RATES):
-                for mi, m in enumerate(mats):
+            ms = ([0] if gated else []) + [1] if phase == 0 else [2]
+            nch = ic if phase == 0 else hc                       # chunks of the output
+            counts = [[len(lists[m][s]) for s in range(MOES_RATES)] for m in ms]
+            for m in ms:
+                for s in range(slots):
                     counts_sh.read((m, s), p, "moeg count")
-                    for li in range(len(lists[m][s])):
-                        lists_sh.read((m, s, li), p, "moeg list")
-                        tid = lists[m][s][li]
-                        rt_sh.read(tid, p, "moeg tile")
-                        e, r0, M = tiles[tid]
-                        rows = slice(r0, r0 + M)             # X rows clamp to M - 1: inside the tile
-                        src = {0: (ts_g, ps["g"]), 1: (ts_u, ps["u"]), 2: (ti_g, ps["d"])}[m]
-                        src[0].read(rows, p, f"moeg A rows (matrix {m})")
-                        src[1].read(rows, p, f"moeg mul1 row sums (matrix {m})")
-                        dst = {0: ti_g, 1: ti_u, 2: ts_g}[m]
-                        dst.write(rows, p)
+            items = lay.rt_cap * len(ms) * nch
+            done = set()
+            for _, i, s, li, chunk in moeg_walk(counts, len(ms), nch, slots, (min(grid, items) + 7) // 8 * 8):
+                m = ms[i]
+                assert 0 <= s < slots and 0 <= li < len(lists[m][s]), "moeg entry outside its list"
+                lists_sh.read((m, s, li), p, "moeg list")
+                tid = lists[m][s][li]
+                assert (m, tid, chunk) not in done, "an item runs twice"
+                done.add((m, tid, chunk))
+                rt_sh.read(tid, p, "moeg tile")
+                e, r0, M = tiles[tid]
+                assert rate_slot(int(Kcodes[m][e])) == s, "a tile runs at its expert's rate"
+                rows = slice(r0, r0 + M)                         # X rows clamp to M - 1: inside the tile
+                src = {0: (ts_g, ps["g"]), 1: (ts_u, ps["u"]), 2: (ti_g, ps["d"])}[m]
+                src[0].read(rows, p, f"moeg A rows (matrix {m})")
+                src[1].read(rows, p, f"moeg mul1 row sums (matrix {m})")
+                {0: ti_g, 1: ti_u, 2: ts_g}[m].write((rows, chunk), p)
+            assert done == {(m, tid, c) for m in ms for tid in range(len(tiles)) for c in range(nch)}, "items left out"
 
         gemm(0)
         # activation: live rows read up (and gate) outputs, write the down input in place

@@ -2,7 +2,8 @@
 configuration of the GPU tests and a seeded sweep of random ones (multi-pass pools of any size,
 experts straddling passes, count ranges, sentinel assignments, empty tokens, mixed and half
 rates, gated and gateless), every read of workspace state or pool rows by the plan, gather,
-grouped GEMM, activation and output kernels hits memory written earlier in the same pass, stale
+grouped GEMM, activation and output kernels hits memory written earlier in the same pass, the grouped
+GEMM's walk over the lists of all rates runs every (row tile, matrix, column chunk) exactly once, stale
 position -> row entries are always rejected by the output kernel's guard, row tiles cover each
 live pool row exactly once, and every in-range assignment reaches the output exactly once.
 """
@@ -25,12 +26,12 @@ GPU_CASES = [
 ]
 
 
-def check(E, H, I, T, topk, Ks, act, max_tok, conc, lo, hi, sentinel, seed, tile_rows=None, tok_mode=True):
+def check(E, H, I, T, topk, Ks, act, max_tok, conc, lo, hi, sentinel, seed, tile_rows=None, tok_mode=True, slots=None,
+          grid=1024, codes=None):
     flat, order, inv, token_sorted, weight_sorted, count, start = routing(T, E, topk, seed=seed, sentinel=sentinel)
-    codes = [rate_code(k) for k in Ks]
-    Kcodes = [codes, codes, codes]
+    Kcodes = codes if codes is not None else [[rate_code(k) for k in Ks]] * 3
     contrib, lay = simulate(count, token_sorted, T, E, H, I, max_tok, conc, lo, hi, Kcodes, gated=act != 2,
-                            tile_rows=tile_rows, tok_mode=tok_mode)
+                            tile_rows=tile_rows, tok_mode=tok_mode, slots=slots, grid=grid)
     # every assignment of an in-range expert contributes once; the rest (sentinel, out of range) never
     exp = np.zeros(len(token_sorted), np.int64)
     for e in range(E):
@@ -52,6 +53,20 @@ def test_gpu_case_index_walk(case, tok_mode):
 def test_tile_sizes_index_walk(tile_rows):
     check(4, 256, 256, 160, 2, [2, 3, 4, 2], 0, 256, 1, 0, 1 << 30, 0, seed=18, tile_rows=tile_rows)
     check(4, 256, 384, 160, 2, [2.5] * 4, 1, 256, 1, 0, 1 << 30, 0, seed=17, tile_rows=tile_rows)
+
+
+@pytest.mark.parametrize("slots", [8, 11])
+@pytest.mark.parametrize("grid", [8, 40, 1024])
+def test_merged_lists_walk(slots, grid):
+    """The lists of all rates in one walk: a different set of rates for each matrix (lists of unequal length
+    side by side), 8 and 11 rate slots, fewer workgroups than items, one matrix set and two."""
+    rng = np.random.default_rng(slots + grid)
+    for it in range(6):
+        E = int(rng.integers(3, 24))
+        rates = (1, 2, 3, 5, 8) if slots == 8 else (1, 4, 17, 18, 19)
+        codes = [[int(rng.choice(rates)) for _ in range(E)] for _ in range(3)]
+        check(E, 256, 384, 60, min(E, 4), None, 2 if it % 2 else 0, 64, 2, 0, 1 << 30, 2, seed=it, slots=slots, grid=grid, codes=codes)
+    check(4, 128, 256, 40, 2, [5] * 4, 0, 64, 1, 0, 1 << 30, 0, seed=1, slots=slots, grid=grid)      # one list
 
 
 def test_edges_index_walk():
