@@ -247,12 +247,7 @@ __device__ __forceinline__ float wave_sum(float v, int lane)
     return v;
 }
 
-// Device-scope loads: they miss the CU's L1 and read the XCD's L2, where the other
-// workgroups of the chunk (same XCD) left their results.
-__device__ __forceinline__ f32x2 load_l2_f32x2(const float* p)
-{
-    return __builtin_bit_cast(f32x2, __hip_atomic_load(to_global((const uint64_t*) p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
+// As load_l2_f32x2.
 __device__ __forceinline__ uint32_t load_l2_u32(const void* p)
 {
     return __hip_atomic_load(to_global((const uint32_t*) p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1310,7 +1305,8 @@ void gemv1b_kernel(const GemvArgs g)
 // (or j + 8) of its own k-tile.  The 8 MFMAs of a unit are (row group gq, column half c):
 // A = the lane's decoded words 8 gq + 4 c .. + 3 (rows 2 gq, 2 gq + 1, 2 gq + 8, 2 gq + 9 of
 // column j + 8 c), B = the input at those rows of the lane's k-tile, read as one 16-byte LDS
-// load from the input staged in that row order (xperm).
+// load from the input staged in that row order: row pairs (2 i, 2 i + 1) and (2 i + 8, 2 i + 9) of a
+// 16-row group side by side ("pair order"; pair i of row half h at pair slot 2 i + h).
 //
 // MUL1 weights are one fp16 each (1024 + byte sum) and come packed in pairs, so their A operands
 // hold 8 weights instead of 4 and the input is staged plain: 4 MFMAs and 2 operand reads per unit
@@ -1322,9 +1318,6 @@ void gemv1b_kernel(const GemvArgs g)
 // kernel's (block_epilogue).
 // ---------------------------------------------------------------------------------------------
 typedef _Float16 f16x8v __attribute__((ext_vector_type(8)));
-
-// position of row rho (0..15) of a 16-row group in the staged input
-__device__ __forceinline__ constexpr int xperm(int rho) { return 4 * ((rho & 7) >> 1) + (rho & 1) + 2 * (rho >> 3); }
 
 template <int K, int CB, int MT>
 __global__ __launch_bounds__(GEMV_THREADS)
@@ -1364,12 +1357,12 @@ void gemvm_kernel(const GemvArgs g)
     constexpr bool PAIRS = CB == 2;
     constexpr int XW = PAIRS ? 8 : 16;                    // u32 per staged row and 16-row k-tile
     const int xs_stride = g.slices_per_block * XW + 4;    // u32 per row; +4: rows 16 bytes apart in the banks
-    uint32_t* xs = smem;                                  // [MT][xs_stride], xperm order
+    uint32_t* xs = smem;                                  // [MT][xs_stride], pair order
     constexpr int RS = 132;                               // res row stride: 16-byte column groups of 16 rows in distinct banks
     float* res = (float*) (smem + MT * xs_stride);        // [MT][RS]
     float* tmp = res + MT * RS;                           // epilogue scratch: 2 x (m x 64 column pairs), >= 512
 
-    // Input rotation of the workgroup's nkc 128-row chunks, every row, into xs (xperm order): 16 lanes
+    // Input rotation of the workgroup's nkc 128-row chunks, every row, into xs (pair order): 16 lanes
     // per (row, chunk) job as had128_kernel, lane g of a job holds rows 8 g .. 8 g + 7, so that a wave
     // rotates 4 jobs in one chain of stages (one job per wave and chain, lane = two rows, took 7.1 us
     // of a 25 us call at 8 rows of 5120 -> 17408).  The first XB steps' input and suh loads are

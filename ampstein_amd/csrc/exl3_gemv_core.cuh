@@ -199,6 +199,13 @@ __device__ __forceinline__ void sum_pairs4(const uint32_t* r, uint32_t* pk)
 #undef EXL3_HI
 }
 
+// Device-scope load: it misses the CU's L1 and reads the XCD's L2, where the other workgroups of this
+// launch (on the same XCD) left their results.
+__device__ __forceinline__ f32x2 load_l2_f32x2(const float* p)
+{
+    return __builtin_bit_cast(f32x2, __hip_atomic_load(to_global((const uint64_t*) p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)

@@ -525,12 +525,6 @@ __device__ __forceinline__ void acquire_handoff(bool xcd)
     else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
-// device-scope load (misses L1): data another workgroup of this launch wrote
-__device__ __forceinline__ f32x2 load_l2_f32x2(const float* p)
-{
-    return __builtin_bit_cast(f32x2, __hip_atomic_load(to_global((const uint64_t*) p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-
 // workgroup -> (chunk, rest): chunk c on XCD c % xcd when enabled
 __device__ __forceinline__ void chunk_coords(int xcd, int chunks, int& chunk, int& rest)
 {

@@ -4,7 +4,8 @@
 // gemm_dma_kernel (which compute 256 rows whatever m is, two waves per SIMD in step) lies the
 // batch of a serving engine: tens of rows.  There the decode of the weights (VALU) is the work,
 // so each weight is decoded once per row tile of 16 R rows, straight into the registers of a
-// matrix operand, and only the row groups that exist are multiplied.
+// matrix operand, and only the row groups that exist are multiplied (there is no instance of 7
+// groups: 97 to 112 rows of a tile run as 8).
 //
 // Work split.  A workgroup owns one 128-column chunk, one row tile and one range of k (split k:
 // S ranges per chunk); its 8 waves are 4 column pairs (two 16-column tiles each) x 2 halves of
@@ -26,7 +27,7 @@
 // unit costs a SIMD ~1100 cycles, of which ~600 are the ~150 VALU instructions of the decode and
 // ~9 per MFMA: on gfx950 a 16x16x32 MFMA holds the VALU for about two issue slots, from whichever
 // wave, so the two add up instead of overlapping; without any memory traffic or barrier the loop
-// takes 840.  Hence one decode per tile, no spare row groups, and little else to gain from deeper
+// takes 840.  Hence one decode per tile, few spare row groups, and little else to gain from deeper
 // rings (4 or 8 units measured the same), interleaving MFMAs with the decode (the same, more
 // registers), or 4 k quarters per workgroup (slower).  Whole call: 36 us against 65 for
 // gemm_dma_kernel with its split k (100 rows of 4096 -> 14336 at 5 bits: 45 against 57; 64 rows
@@ -86,11 +87,6 @@ __device__ __forceinline__ void decode_pairs(const uint32_t* wv, uint32_t* pk, u
         }
         __builtin_amdgcn_sched_barrier(0);
     });
-}
-
-__device__ __forceinline__ f32x2 load_l2_pair(const float* p)
-{
-    return __builtin_bit_cast(f32x2, __hip_atomic_load(to_global((const uint64_t*) p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
 template <int K, int CB, int R>
@@ -276,7 +272,7 @@ void rows_kernel(const RowsArgs g)
             {
                 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    v[i][q] = load_l2_pair(pb + (size_t) min(p0 + q, S - 1) * (RT * 128) + min(r0 + RW * i, M - 1) * 128 + 2 * lane);
+                    v[i][q] = load_l2_f32x2(pb + (size_t) min(p0 + q, S - 1) * (RT * 128) + min(r0 + RW * i, M - 1) * 128 + 2 * lane);
             }
             #pragma unroll
             for (int i = 0; i < 4; ++i)
