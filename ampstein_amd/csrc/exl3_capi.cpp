@@ -963,9 +963,11 @@ int exl3_amd_to_slabs(const uint16_t* x, uint16_t* y, int rows, int cols, int ro
 
 namespace {
 
-// The kernels that stage rows with global_load_lds_dwordx4 take them from 16-byte aligned addresses
+// The kernels that stage rows with 16-byte LDS DMAs take them from 16-byte aligned addresses
 // only; plain loads take any.  Rows are multiples of 256 bytes, so the base decides.
 bool dma_aligned(const void* p) { return ((uintptr_t) p & 15) == 0; }
+// Their 128-row tiles are addressed with 32-bit byte offsets.
+constexpr int DMA_MAX_K = 1 << 22;
 
 // exl3_gemm on a given workspace (the library's per-device one, or the no-alloc scratch).
 // ws == nullptr: the library's, set up on first use.
@@ -1486,7 +1488,8 @@ int exl3_amd_moe(const uint16_t* hidden_state, int bsz, int hidden_dim, float* o
     // expert for most experts
     // (the LDS-tiled one also where moeg's LDS DMA cannot take the caller's row buffers)
     const bool reg_gemm = policy(EXL3_AMD_POLICY_MOE_GEMM) != EXL3_AMD_MOE_GEMM_LDS && dma_aligned(temp_state_g) &&
-                          dma_aligned(temp_state_u) && dma_aligned(temp_intermediate_g);
+                          dma_aligned(temp_state_u) && dma_aligned(temp_intermediate_g) &&
+                          hidden_dim <= DMA_MAX_K && intermediate_dim <= DMA_MAX_K;
     // moeg: the smallest tile holding ~1.5x the mean rows (the largest expert, for top-k routing
     // of random tokens).  Measured, 256 experts 4096 -> 2048 -> 4096, top-8: T = 512 (mean 16,
     // max 27) best at 32 or 64 (0.99 / 1.07 ms); T = 1024 (mean 32) at 64: 1.19 against 1.48 at 32 and

@@ -221,17 +221,30 @@ __device__ __forceinline__ uint32_t win_reg(const uint32_t* wv)
 // tile (lane 0: the ring wraps to the tile's last word), shifted left by 16 bits for even j so
 // that the frame starts at word 0, bit 0 (MSB-first).
 template <int K>
-__device__ __forceinline__ void load_frame_half(const uint32_t* __restrict__ tile, int j, uint32_t* wv)
+__device__ __forceinline__ void load_frame_raw(const uint32_t* __restrict__ tile, int j, uint32_t* raw)
 {
     constexpr int B = kbits(K);
     const int b = j * B + (j >> 1) - 1;
-    uint32_t raw[B + 2];
     raw[0] = __builtin_nontemporal_load(to_global(tile) + (b < 0 ? tile_words(K) - 1 : b));
     #pragma unroll
     for (int i = 1; i < B + 2; ++i) raw[i] = __builtin_nontemporal_load(to_global(tile) + b + i);
+}
+
+// raw's b + 2 words -> the frame's b + 1 (wv may be raw).
+template <int K>
+__device__ __forceinline__ void shift_frame(const uint32_t* raw, int j, uint32_t* wv)
+{
     const uint32_t sh = (j & 1) ? 0u : 16u;
     #pragma unroll
-    for (int i = 0; i <= B; ++i) wv[i] = __builtin_amdgcn_alignbit(raw[i], raw[i + 1], sh);
+    for (int i = 0; i <= kbits(K); ++i) wv[i] = __builtin_amdgcn_alignbit(raw[i], raw[i + 1], sh);
+}
+
+template <int K>
+__device__ __forceinline__ void load_frame_half(const uint32_t* __restrict__ tile, int j, uint32_t* wv)
+{
+    uint32_t raw[kbits(K) + 2];
+    load_frame_raw<K>(tile, j, raw);
+    shift_frame<K>(raw, j, wv);
 }
 
 // Decode the lane's 32 windows into 16 packed pairs: out[q] = (window 2q, window 2q+1).

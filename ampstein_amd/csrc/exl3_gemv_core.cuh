@@ -74,6 +74,21 @@ __device__ __forceinline__ void load_tile_lane(const uint32_t* __restrict__ tile
     else load_slot<K>(tile + j * K, prev_off, w);
 }
 
+// The same load as it comes: half rates keep their b + 2 raw words, which ring_words shifts into the frame
+// when the slot is used (a shift behind the loads would wait for them there).
+template <int K> constexpr int RING_WORDS = kbits(K) + (khalf(K) ? 2 : 1);
+template <int K>
+__device__ __forceinline__ void load_tile_ring(const uint32_t* __restrict__ tile, int j, int prev_off, uint32_t* w)
+{
+    if constexpr (khalf(K)) load_frame_raw<K>(tile, j, w);
+    else load_slot<K>(tile + j * K, prev_off, w);
+}
+template <int K>
+__device__ __forceinline__ void ring_words(uint32_t* w, int j)
+{
+    if constexpr (khalf(K)) shift_frame<K>(w, j, w);
+}
+
 // Clean 16-bit state of window I (exl3_common.cuh: Win): one bfe, from word hi when the window
 // sits inside it, else from the half-word-shifted word alignbit(wv[hi-1], wv[hi], 16) (one per
 // word, shared by the windows that straddle that word boundary).
@@ -208,10 +223,19 @@ __device__ __forceinline__ f32x2 load_l2_f32x2(const float* p)
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
+// Buffer resource over `bytes` bytes from p (both the same in every lane): LDS DMAs through it take 32-bit
+// lane offsets.  Where a loop also holds loads in registers, its DMAs go this way: global_load_lds
+// counts as a flat access of both memories, and while one is in flight the compiler waits for all
+// loads (vmcnt(0)) wherever any is used.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((void*) p, (short) 0, (int) bytes, 0x00020000);
+}
+
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
 #define EXL3_WAIT_VM_LGKM0(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4))
 
-// Fewest vector-memory instructions that load_tile_lane<K> compiles to (neighbouring words may
+// Fewest vector-memory instructions that load_tile_ring<K> compiles to (neighbouring words may
 // be loaded together): the row waits count on at least this many per unit.
 constexpr int tile_lane_loads(int K) { return khalf(K) ? 2 : (K + 3) / 4 + 1; }
 

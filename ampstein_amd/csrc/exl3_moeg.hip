@@ -19,7 +19,7 @@
 // sum(x) from the 128-chunk sums the staging kernels write beside the rows (psum, added in a
 // fixed order).  MCG weights are the reference's fp16 lo + hi (one rounding).
 //
-// The rows go from L2 into LDS with global_load_lds_dwordx4, MG_XD units ahead; one barrier per
+// The rows go from L2 into LDS with buffer_load_dwordx4 ... lds, MG_XD units ahead; one barrier per
 // unit publishes its rows and frees the previous unit's.
 //
 // One launch takes every bitrate: the item finds its list (and so its rate) on the device, and the
@@ -27,9 +27,15 @@
 // (blockIdx % 8) take the (row tile, matrix) entries e with e % 8 == x, so all chunks of an entry
 // share one L2.  Measured on MI355X against one launch per possible bitrate (8 with rate tables, most
 // of them without an entry, each with a tail of its own), mul1 at 2, 3 and 4 bits, whole calls: 16
-// experts 3072 -> 1024, 300 tokens, top-2: 67 -> 38 us; 64 experts 2048 -> 1536, 512 tokens, top-4: 290 ->
-// 193; 128 experts 2048 -> 1024, 4096 tokens, top-8: 1196 -> 1042; 256 experts 4096 -> 2048, top-8:
-// 2048 tokens 1762 -> 1650, 1024 tokens 1241 -> 1201, 512 tokens 1016 -> 1010.
+// experts 3072 -> 1024, 300 tokens, top-2: 210 -> 91 us; 64 experts 2048 -> 1536, 512 tokens, top-4: 269 ->
+// 158; 128 experts 2048 -> 768, 4096 tokens, top-8: 989 -> 750; 256 experts 4096 -> 2048, top-8:
+// 2048 tokens 1806 -> 1462, 1024 tokens 1244 -> 1067, 512 tokens 985 -> 931.  At one rate, where that was
+// one launch too: 64 experts 2048 -> 1536, 512 tokens, at 4 / 2.5 bits 173 -> 160 / 171 -> 157.
+//
+// The trellis loads of two units and the row DMAs of two stay in flight across the barrier.  That takes DMAs
+// through a buffer resource, a single LDS array and half-rate words that are shifted when they are used;
+// with global_load_lds, several LDS variables and a shift at the load the compiler waited for everything
+// once a unit, and at one rate the calls took 8 to 28 % longer at 2.5 bits, up to 34 % with few experts.
 //
 // What bounds it: the issue slots.  A unit is 96 VALU instructions of decode (bfe, mul, sad a weight)
 // per 10 MFMAs at 40 rows; the counters show 61 % of the cycles issuing VALU and 21 % in MFMAs, which
@@ -105,34 +111,35 @@ __device__ __forceinline__ void moeg_sums(const uint16_t* A, int M, int k, int t
     const uint32_t* tile0 = trellis + ((size_t) (lane >> 4) * tiles_n + chunk * 8 + 2 * wave + ((lane >> 3) & 1)) * TWD;
     const size_t ustride = (size_t) 4 * tiles_n * TWD;
     const int prev_off = jt == 0 ? 8 * KB - 1 : -1;
-    uint32_t ring[PF][KB + 1];
+    uint32_t ring[PF][RING_WORDS<K>];
 
     // Row staging: a unit is 2 G blocks of 8 rows x 128 bytes; wave w fills blocks w, w + 4, ... (past the
     // last one: the same bytes to the same place, so that every wave issues the same number).  Rows
     // past M repeat row M - 1; their products are never stored.  16-byte chunk c of row r sits at
     // chunk c ^ s(r % 16), s(q) = (q ^ (q >> 3)) & 7: no bank conflicts for the operand reads.
     constexpr int ND = (2 * G + 3) / 4;
-    const uint16_t* xsrc[ND];
+    const __amdgpu_buffer_rsrc_t rows = buffer_of(A, (uint32_t) (M * k * 2));
+    uint32_t xoff[ND];
     #pragma unroll
     for (int i = 0; i < ND; ++i)
     {
         const int q = min(wave + 4 * i, 2 * G - 1), row = 8 * q + (lane >> 3), rr = row & 15;
-        xsrc[i] = A + (size_t) min(row, M - 1) * k + 8 * ((lane & 7) ^ ((rr ^ (rr >> 3)) & 7));
+        xoff[i] = (uint32_t) (2 * (min(row, M - 1) * k + 8 * ((lane & 7) ^ ((rr ^ (rr >> 3)) & 7))));
     }
     auto xissue = [&](int u) {
         #pragma unroll
         for (int i = 0; i < ND; ++i)
         {
             const int q = min(wave + 4 * i, 2 * G - 1);
-            __builtin_amdgcn_global_load_lds((const void*) (xsrc[i] + min(u, units - 1) * 64),
-                                             (lds_ptr_t) (lds + (u % MG_XNB) * XBUF + 256 * q), 16, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_ptr_t) (lds + (u % MG_XNB) * XBUF + 256 * q), 16, xoff[i],
+                                                     (uint32_t) (min(u, units - 1) * 128), 0, 0);
         }
     };
     // issue order: rows(0), trellis(0), rows(1), trellis(1), ...; then per unit rows(u + XD), trellis(u + PF)
     static_for<0, (PF > MG_XD ? PF : MG_XD)>([&](auto d) {
         if constexpr (d < MG_XD) xissue(d);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (d < PF) load_tile_lane<K>(tile0 + (size_t) min((int) d, units - 1) * ustride, jt, prev_off, ring[d]);
+        if constexpr (d < PF) load_tile_ring<K>(tile0 + (size_t) min((int) d, units - 1) * ustride, jt, prev_off, ring[d]);
         __builtin_amdgcn_sched_barrier(0);
     });
     f32x4 acc[2][G];
@@ -153,6 +160,7 @@ __device__ __forceinline__ void moeg_sums(const uint16_t* A, int M, int k, int t
         // a row half at a time (registers): its row operands first (their LDS latency hides behind the
         // decode), its pairs, its products
         const uint32_t* xs = lds + d * XBUF;
+        ring_words<K>(ring[d % PF], jt);
         static_for<0, 2>([&](auto hh) {
             constexpr int h = hh;
             h8v bx[G];
@@ -162,7 +170,7 @@ __device__ __forceinline__ void moeg_sums(const uint16_t* A, int M, int k, int t
             uint32_t pk[8];
             moeg_pairs<K, CB, h>(ring[d % PF], pk);
             if constexpr (h == 1)
-                load_tile_lane<K>(tile0 + (size_t) min(u + PF, units - 1) * ustride, jt, prev_off, ring[d % PF]);
+                load_tile_ring<K>(tile0 + (size_t) min(u + PF, units - 1) * ustride, jt, prev_off, ring[d % PF]);
             __builtin_amdgcn_sched_barrier(0);
             #pragma unroll
             for (int r = 0; r < G; ++r)
@@ -182,6 +190,13 @@ __device__ __forceinline__ void moeg_sums(const uint16_t* A, int M, int k, int t
     for (; u + 4 <= units; u += 4) static_for<0, 4>([&](auto d) { unit(u + d, d); });
     if (u < units) static_for<0, 2>([&](auto d) { unit(u + d, d); });      // (units is even)
     EXL3_WAIT_VM_LGKM0(0);                                // the past-the-end row loads still write LDS
+    // the past-the-end trellis loads have to stay: the row waits count them
+    #pragma unroll
+    for (int d = 0; d < PF; ++d)
+    {
+        #pragma unroll
+        for (int w = 0; w < RING_WORDS<K>; ++w) asm volatile("" :: "v"(ring[d][w]));
+    }
     __syncthreads();
     // D[i][nn] of acc[c][r] (lane: i = 4 (lane / 16) + e, nn = lane % 16) is column
     // 32 w + 16 (i / 8) + i % 8 + 8 c, row 16 r + nn
@@ -212,9 +227,11 @@ __attribute__((amdgpu_waves_per_eu(moeg_waves(R), moeg_waves(R))))
 void moeg_kernel(const MoegArgs g)
 {
     using LD = MgLds<R>;
-    __shared__ __align__(16) uint32_t lds[LD::TOTAL];
-    __shared__ int ends[64];
-    __shared__ float sumx[LD::RT];
+    // one array: with a second LDS variable in the kernel the compiler tracks the DMAs into this one and waits
+    // for all of them (vmcnt(0)) before any read of it; the unit loop's own waits are what orders them
+    __shared__ __align__(16) uint32_t lds[LD::TOTAL + 64 + LD::RT];
+    int* ends = (int*) (lds + LD::TOTAL);
+    float* sumx = (float*) (lds + LD::TOTAL + 64);
     const int t = threadIdx.x, lane = t & 63;
     const int k = g.k, n = g.n;
     const int nch = n / 128;
@@ -248,8 +265,9 @@ void moeg_kernel(const MoegArgs g)
         const int s = __builtin_popcountll(before), slot = g.slots - 1 - s;
         const int li = pos - (s ? __builtin_amdgcn_readfirstlane(ends[32 * mat + s - 1]) : 0);
         const int tid = *to_global((mat ? g.list[1] : g.list[0]) + (size_t) slot * g.list_stride + li);
-        const int e = *to_global(g.rt + 3 * tid), row0 = *to_global(g.rt + 3 * tid + 1);
-        const int M = *to_global(g.rt + 3 * tid + 2);
+        const int e = *to_global(g.rt + 3 * tid);
+        const int row0 = __builtin_amdgcn_readfirstlane(*to_global(g.rt + 3 * tid + 1));
+        const int M = __builtin_amdgcn_readfirstlane(*to_global(g.rt + 3 * tid + 2));
         const uint16_t* A = (mat ? g.A[1] : g.A[0]) + (size_t) row0 * k;
         uint16_t* C = (mat ? g.C[1] : g.C[0]) + (size_t) row0 * n + chunk * 128;
         const uint32_t* trellis = (const uint32_t*) *to_global((mat ? g.tab[1] : g.tab[0]) + e);
