@@ -1051,7 +1051,7 @@ int gemm_impl(const Workspace* ws, const uint16_t* A, const uint16_t* trellis, v
         rr.m = m; rr.k = k; rr.n = n; rr.c_fp32 = c_fp32 ? 1 : 0;
         const double t_rows = rows_plan(*ws, m, k, n, rr);
         const bool rows = policy(EXL3_AMD_POLICY_GEMM_KERNEL) == EXL3_AMD_GEMM_KERNEL_ROWS || (t_rows <= t_gemm && t_rows <= t_group);
-        if (staging == 0 && rows)
+        if (staging == 0 && rows && k <= DMA_MAX_K)
         {
             int rc = dispatch_rows(bits, cb, rr, s);
             if (rc) return hip_fail(rc, name);

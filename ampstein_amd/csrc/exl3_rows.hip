@@ -15,23 +15,23 @@
 // and row half h is pairs { h, 4 + h, 8 + h, 12 + h } + 2 c; operand B (32 k x 16 rows) is 16
 // contiguous bytes of an input row: k 64 u + 16 (lane / 16) + 8 h .. + 7, from LDS.
 //
-// The rotated rows go from L2 into LDS with global_load_lds_dwordx4, ROWS_XD units ahead, 8 rows x
+// The rotated rows go from L2 into LDS with buffer_load_dwordx4 ... lds, ROWS_XD units ahead, 8 rows x
 // 128 bytes (whole lines) per instruction; lane -> chunk is permuted so that the operand reads
 // are conflict-free.  One barrier per unit: it publishes unit u's rows and frees unit u - 1's.
 //
 // Numerics are the tiled GEMM's: the reference's fp16 weights (3INST / MCG: lo + hi, MUL1: one fma,
 // one rounding each), fp32 accumulation, output rotation in fp32.
 //
-// What bounds it (MI355X, 33 rows of 17408 -> 5120 at 4 bits, wave timestamps): of 31 us, 24 are
-// the unit loop, 1.3 the fill, 1.5 the reduction, 2.8 the last arrival's sum and rotation.  A
-// unit costs a SIMD ~1100 cycles, of which ~600 are the ~150 VALU instructions of the decode and
-// ~9 per MFMA: on gfx950 a 16x16x32 MFMA holds the VALU for about two issue slots, from whichever
-// wave, so the two add up instead of overlapping; without any memory traffic or barrier the loop
-// takes 840.  Hence one decode per tile, few spare row groups, and little else to gain from deeper
-// rings (4 or 8 units measured the same), interleaving MFMAs with the decode (the same, more
-// registers), or 4 k quarters per workgroup (slower).  Whole call: 36 us against 65 for
-// gemm_dma_kernel with its split k (100 rows of 4096 -> 14336 at 5 bits: 45 against 57; 64 rows
-// of 14336 -> 4096: 31 against 53).
+// What bounds it: the decode's VALU instructions (~134 a unit) and the MFMAs, which add up on a SIMD: on
+// gfx950 a 16x16x32 MFMA holds the VALU for about two issue slots, from whichever wave.  Hence one
+// decode per tile and few spare row groups; interleaving MFMAs with the decode or 4 k quarters per
+// workgroup gained nothing.  The trellis loads of two units and the row DMAs of two stay in flight across the
+// barrier: the DMAs go through a buffer resource, LDS is one array and half-rate words are shifted when
+// used.  With global_load_lds, a second LDS variable and a shift at the load the compiler waited for every
+// load once or twice a turn of the buffers.  MI355X, whole calls before / after, us: 32 rows of 17408 ->
+// 5120 at 4 / 3.5 bits 34.7 / 28.3 and 35.8 / 27.9, 9 rows of 8192 -> 28672 at 4 bits 66.4 / 48.0 (the GEMV of
+// 16-row groups: 62 to 67), 64 rows of 14336 -> 4096 31.8 / 27.8, 96 rows of 4096 -> 14336 34.9 / 31.6.
+// gemm_dma_kernel with its split k: 65 us for 33 rows of 17408 -> 5120, 57 for 100 rows of 4096 -> 14336.
 //
 // Split k: each range stores its fp32 partial rows; the last arrival of a chunk (XCD-local
 // hand-off, exl3_xcd.cuh) adds them in k order, four rows in flight per wave, rotates and stores.
@@ -89,15 +89,13 @@ __device__ __forceinline__ void decode_pairs(const uint32_t* wv, uint32_t* pk, u
     });
 }
 
+// rows_kernel's body (a device function: the host pass knows no buffer resources).
 template <int K, int CB, int R>
-__global__ __launch_bounds__(ROWS_THREADS)
-__attribute__((amdgpu_waves_per_eu(R <= 4 ? 4 : 2, R <= 4 ? 4 : 2)))
-void rows_kernel(const RowsArgs g)
+__device__ __forceinline__ void rows_body(const RowsArgs& g, uint32_t* lds)
 {
     using LD = RowsLds<R>;
     constexpr int TWD = tile_words(K), KB = kbits(K), RT = LD::RT, XBUF = RT * 32;
-    __shared__ __align__(16) uint32_t lds[LD::TOTAL];
-    __shared__ int flag;
+    int* flag = (int*) (lds + LD::TOTAL);
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int cw = wave & 3, kg = wave >> 2;              // column pair, k half
@@ -116,7 +114,7 @@ void rows_kernel(const RowsArgs g)
                           + ((size_t) (u00 * 4 + (lane >> 4)) * tiles_n + chunk * 8 + 2 * cw + ((lane >> 3) & 1)) * TWD;
     const size_t ustride = (size_t) 4 * tiles_n * TWD;
     const int prev_off = jt == 0 ? 8 * KB - 1 : -1;
-    uint32_t ring[ROWS_PF][KB + 1];
+    uint32_t ring[ROWS_PF][RING_WORDS<K>];
 
     // Row staging: a unit is 2 R blocks of 8 rows x 128 bytes; wave cw of the k half fills blocks
     // cw, cw + 4, ... (past the last one: the same bytes to the same place, so that every wave
@@ -124,27 +122,28 @@ void rows_kernel(const RowsArgs g)
     // 16-byte chunk c of row r sits at chunk c ^ s(r % 16), s(q) = (q ^ (q >> 3)) & 7 (moeg_kernel's).
     constexpr int ND = (2 * R + 3) / 4;
     uint32_t* xs = lds + kg * (ROWS_XNB * XBUF);
-    const uint16_t* xsrc[ND];
+    const __amdgpu_buffer_rsrc_t rows = buffer_of(A, (uint32_t) (2 * ((M - 1) * k + units * 64)));
+    uint32_t xoff[ND];
     #pragma unroll
     for (int i = 0; i < ND; ++i)
     {
         const int q = min(cw + 4 * i, 2 * R - 1), row = 8 * q + (lane >> 3), rr = row & 15;
-        xsrc[i] = A + (size_t) min(row, M - 1) * k + 8 * ((lane & 7) ^ ((rr ^ (rr >> 3)) & 7));
+        xoff[i] = (uint32_t) (2 * (min(row, M - 1) * k + 8 * ((lane & 7) ^ ((rr ^ (rr >> 3)) & 7))));
     }
     auto xissue = [&](int u) {
         #pragma unroll
         for (int i = 0; i < ND; ++i)
         {
             const int q = min(cw + 4 * i, 2 * R - 1);
-            __builtin_amdgcn_global_load_lds((const void*) (xsrc[i] + min(u, units - 1) * 64),
-                                             (lds_ptr_t) (xs + (u % ROWS_XNB) * XBUF + 256 * q), 16, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_ptr_t) (xs + (u % ROWS_XNB) * XBUF + 256 * q), 16, xoff[i],
+                                                     (uint32_t) (min(u, units - 1) * 128), 0, 0);
         }
     };
     // issue order: rows(0), trellis(0), rows(1), trellis(1), rows(2); then per unit trellis(u + PF), rows(u + XD)
     static_for<0, ROWS_XD>([&](auto d) {
         xissue(d);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (d < ROWS_PF) load_tile_lane<K>(tile0 + (size_t) min((int) d, units - 1) * ustride, jt, prev_off, ring[d]);
+        if constexpr (d < ROWS_PF) load_tile_ring<K>(tile0 + (size_t) min((int) d, units - 1) * ustride, jt, prev_off, ring[d]);
         __builtin_amdgcn_sched_barrier(0);
     });
 
@@ -160,8 +159,9 @@ void rows_kernel(const RowsArgs g)
             const int u = u0 + d;
             if (u >= units) break;
             uint32_t pk[16];
+            ring_words<K>(ring[d % ROWS_PF], jt);
             decode_pairs<K, CB>(ring[d % ROWS_PF], pk, a3, b3);
-            load_tile_lane<K>(tile0 + (size_t) min(u + ROWS_PF, units - 1) * ustride, jt, prev_off, ring[d % ROWS_PF]);
+            load_tile_ring<K>(tile0 + (size_t) min(u + ROWS_PF, units - 1) * ustride, jt, prev_off, ring[d % ROWS_PF]);
             __builtin_amdgcn_sched_barrier(0);
             // unit u's rows have landed when all but the row loads of units u + 1, u + 2 and the trellis
             // loads issued after unit u's rows are done (loads complete in issue order)
@@ -199,6 +199,13 @@ void rows_kernel(const RowsArgs g)
         }
     }
     EXL3_WAIT_VM_LGKM0(0);                                     // the past-the-end row loads still write LDS
+    // the past-the-end trellis loads have to stay: the row waits count them
+    #pragma unroll
+    for (int d = 0; d < ROWS_PF; ++d)
+    {
+        #pragma unroll
+        for (int w = 0; w < RING_WORDS<K>; ++w) asm volatile("" :: "v"(ring[d][w]));
+    }
     __syncthreads();
 
     // the k halves meet in LDS: D[i][nn] of acc[c][r] (lane: i = 4 (lane / 16) + e, nn = lane % 16) is
@@ -257,9 +264,9 @@ void rows_kernel(const RowsArgs g)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
-    if (t == 0) flag = xcd_arrive(g.xg, g.ctr + tile * 32, S);
+    if (t == 0) *flag = xcd_arrive(g.xg, g.ctr + tile * 32, S);
     __syncthreads();
-    if (!flag) return;
+    if (!*flag) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     for (int r0 = wave; r0 < M; r0 += 4 * RW)
     {
@@ -286,6 +293,17 @@ void rows_kernel(const RowsArgs g)
         for (int i = 0; i < 4; ++i)
             if (r0 + RW * i < M) gemm_store(s0[i], s1[i], g.C, g.c_fp32, has_svh, svp, c0 + (size_t) (r0 + RW * i) * n, lane);
     }
+}
+
+template <int K, int CB, int R>
+__global__ __launch_bounds__(ROWS_THREADS)
+__attribute__((amdgpu_waves_per_eu(R <= 4 ? 4 : 2, R <= 4 ? 4 : 2)))
+void rows_kernel(const RowsArgs g)
+{
+    // one array: with a second LDS variable in the kernel the compiler tracks the DMAs into this one and waits
+    // for all of them (vmcnt(0)) before any read of it; the unit loop's own waits are what orders them
+    __shared__ __align__(16) uint32_t lds[RowsLds<R>::TOTAL + 4];
+    rows_body<K, CB, R>(g, lds);
 }
 
 template <int K, int CB, int R>

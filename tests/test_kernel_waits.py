@@ -40,7 +40,8 @@ def units(src, defines, kernel, tmp_path):
 
 @pytest.mark.parametrize("src,defines,kernel,ahead", [
     ("exl3_moeg.hip", ["-DEXL3_MOEG_CB=2", "-DEXL3_MOEG_R=2"], "moeg_kernel", (2, 2)),
-    ("exl3_moeg.hip", ["-DEXL3_MOEG_CB=1", "-DEXL3_MOEG_R=6"], "moeg_kernel", (2, 2))])
+    ("exl3_moeg.hip", ["-DEXL3_MOEG_CB=1", "-DEXL3_MOEG_R=6"], "moeg_kernel", (2, 2)),
+    ("exl3_rows.hip", ["-DEXL3_INST_K=5"], "rows_kernel", (2, 3)), ("exl3_rows.hip", ["-DEXL3_INST_K=18"], "rows_kernel", (2, 3))])
 def test_unit_waits(src, defines, kernel, ahead, tmp_path):
     """ahead: units whose row DMAs and whose weight loads the row wait leaves in flight."""
     found = units(src, defines, kernel, tmp_path)
