@@ -589,7 +589,9 @@ def pmc_child(workload="decode"):
       moe     -- exl3_moe_coop, 256 experts, 16 tokens, twice;
       moes    -- the token-sorted exl3_moe on the same experts, T = 512 and 2048;
       qwenm   -- the row-batched matrix-core GEMV (gemvm_kernel) on the configs[2] shapes 5120 -> 17408
-                 and 17408 -> 5120, K = 4 3INST, M = 4 and 8, twice each."""
+                 and 17408 -> 5120, K = 4 3INST, M = 4 and 8, twice each;
+      rows    -- the row-tile GEMM (rows_kernel): 33 rows of 17408 -> 5120 and 100 rows of 4096 -> 14336
+                 (K = 4 3INST), 64 rows of 14336 -> 4096 (K = 3.5 mul1), twice each."""
     import torch
     from ampstein_amd import ops, bundles
     torch.cuda.set_device(0)
@@ -653,6 +655,13 @@ def pmc_child(workload="decode"):
                 C = torch.empty((m, n), dtype=torch.half, device="cuda")
                 for _ in range(2):
                     ops.exl3_gemm(x, t, C, s, torch.empty_like(x), v)
+    elif workload == "rows":
+        for si, (m, k, n, K) in enumerate(((33, 17408, 5120, 4), (100, 4096, 14336, 4), (64, 14336, 4096, 3.5))):
+            t, s, v = host_trellis(torch, k, n, K, 6000 + si)
+            x = host_normal(torch, (m, k), 6010 + m)
+            C = torch.empty((m, n), dtype=torch.half, device="cuda")
+            for _ in range(2):
+                ops.exl3_gemm(x, t, C, s, torch.empty_like(x), v, 0, False, K == 3.5)
     torch.cuda.synchronize()
     return 0
 
@@ -679,7 +688,7 @@ def summarize_pmc(outdirs):
             with open(path) as f:
                 for r in csv.DictReader(f):
                     name = r["Kernel_Name"]
-                    if not any(key in name for key in ("gemv", "gemm", "moe_", "moes_", "moeg", "reconstruct", "had128", "copy", "Copy", "Cijk")):
+                    if not any(key in name for key in ("gemv", "gemm", "rows_", "moe_", "moes_", "moeg", "reconstruct", "had128", "copy", "Copy", "Cijk")):
                         continue
                     key = (name.replace("(anonymous namespace)::", "").split("(")[0][:80], r.get("Grid_Size", ""))
                     d = acc.setdefault(key, {}).setdefault(r["Counter_Name"], {})
@@ -771,7 +780,7 @@ def summarize_trace(path, gap_ms=0.0):
     with open(path) as f:
         for r in csv.DictReader(f):
             name = r["Kernel_Name"]
-            if not any(key in name for key in ("gemv", "reconstruct", "had128", "gemm", "moe_", "moes_", "moeg", "rms_norm",
+            if not any(key in name for key in ("gemv", "reconstruct", "had128", "gemm", "rows_", "moe_", "moes_", "moeg", "rms_norm",
                                                "silu_mul", "res_sq", "norm_sq", "Cijk")):
                 continue
             grid = (r.get("Grid_Size_X") or r.get("Grid_Size"), r.get("Grid_Size_Y", "1"))
@@ -802,11 +811,13 @@ RATE_OPS = ["v_bfe_u32", "v_mad_u64_u32", "v_bitop3_b32", "v_mad_u32_u16", "v_pe
 
 def recon_rows():
     """Prefill and medium-batch routes by row count (4 bpw 3INST unless noted, x N(0,1)): per shape
-    and rows, us per call of exl3_gemm as 16-row GEMV groups (force_shape_idx 1, up to 192 rows),
-    exl3_gemm on the MFMA GEMM (force 2: k split when its tiles fill at most half the CUs), the
+    and rows, us per call of exl3_gemm as its own time models route it, as 16-row GEMV groups
+    (force_shape_idx 1, up to 192 rows), on the row tiles (policy EXL3_AMD_POLICY_GEMM_KERNEL, up to 768
+    rows) and on the tiled MFMA GEMM (force 2: k split when its tiles fill at most half the CUs), the
     recon route's rotated branch (exl3_gemm_recon: x rotation, reconstruct, dense GEMM with its own
-    split k) and the same route without the split (policy EXL3_AMD_RECON_MM_NO_SPLIT).  One JSON
-    line per shape; null where a route is not timed."""
+    split k) and the same route without the split (policy EXL3_AMD_RECON_MM_NO_SPLIT).  145 to 768 rows
+    hold both sides of LinearEXL3's switch at 512.  One JSON line per shape; null where a route is
+    not timed."""
     import torch
     from ampstein_amd import ops, _lib
     torch.cuda.set_device(0)
@@ -815,17 +826,20 @@ def recon_rows():
               (8192, 28672, 4), (28672, 8192, 4))
     for si, (k, n, K) in enumerate(shapes):
         t, s, v = host_trellis(torch, k, n, K, 7000 + si)
-        row = {"shape": f"{k}x{n}", "K": K, "us": "gemv groups / mfma gemm / recon (split k) / recon (no split)"}
-        for m in (16, 32, 64, 128, 192, 512, 2048):
+        row = {"shape": f"{k}x{n}", "K": K, "us": "own choice / gemv groups / row tiles / tiled gemm / recon (split k) / recon (no split)"}
+        for m in (16, 32, 64, 128, 145, 192, 256, 384, 512, 768, 2048):
             x = host_normal(torch, (m, k), 7100 + m)
             C = torch.empty((m, n), dtype=torch.half, device="cuda")
             ah = torch.empty_like(x)
-            g = timed(torch, lambda: ops.exl3_gemm(x, t, C, s, ah, v, 1)) if m <= 192 else None
-            f = timed(torch, lambda: ops.exl3_gemm(x, t, C, s, ah, v, 2))
-            r = timed(torch, lambda: ops.exl3_gemm_recon(x, t, s, v, float(K), fused_rows=1 << 30))
+            us = [timed(torch, lambda: ops.exl3_gemm(x, t, C, s, ah, v))]
+            us.append(timed(torch, lambda: ops.exl3_gemm(x, t, C, s, ah, v, 1)) if m <= 192 else None)
+            with _lib.policy(_lib.POLICY_GEMM_KERNEL, _lib.GEMM_KERNEL_ROWS):
+                us.append(timed(torch, lambda: ops.exl3_gemm(x, t, C, s, ah, v)) if m <= 768 else None)
+            us.append(timed(torch, lambda: ops.exl3_gemm(x, t, C, s, ah, v, 2)))
+            us.append(timed(torch, lambda: ops.exl3_gemm_recon(x, t, s, v, float(K), fused_rows=1 << 30)))
             with _lib.policy(_lib.POLICY_RECON_MM, _lib.RECON_MM_NO_SPLIT):
-                r0 = timed(torch, lambda: ops.exl3_gemm_recon(x, t, s, v, float(K), fused_rows=1 << 30))
-            row[str(m)] = [None if g is None else round(g, 1), round(f, 1), round(r, 1), round(r0, 1)]
+                us.append(timed(torch, lambda: ops.exl3_gemm_recon(x, t, s, v, float(K), fused_rows=1 << 30)))
+            row[str(m)] = [None if u is None else round(u, 1) for u in us]
         print(json.dumps(row), flush=True)
         del t, s, v
         torch.cuda.empty_cache()
