@@ -346,18 +346,30 @@ int gemv_plan(int m, int k, int n, int bszm, int num_cus, GemvArgs& g, size_t pa
             // rotation; a workgroup alone on its CU hides less: 1.65), 0.5 us per workgroup, and
             // with S > 1 the hand-off and the last arrival's sum.  Ranges need not divide k evenly:
             // 5120 x 5120 at 8 rows takes S = 12 (480 workgroups), 13.9 us with S = 10 before.
+            // With an index list or per-matrix widths (column slices are all as wide as they say) many workgroups
+            // may have no work, which the model counts as if they had: there a range of up to 4 rows is at
+            // most 8 chunks long, so that the others are enough by themselves.  2 rows at 4 bits, us with that /
+            // with the model's S alone: 4 of 32 slots of 4096 -> 1536 14.0 / 20.8, 1 of 8 of 4096 -> 14336 15.5 /
+            // 20.2, widths 14336 and 7 x 128 of 4096 23.5 / 33.0; every slot in use, 8 of 4096 -> 4096 25.4 /
+            // 26.0.  (Above 4 rows the staged rows allow 11 chunks at most, and 8 would cost full lists more,
+            // 8 of 4096 -> 4096 at 8 rows 32.6 / 28.0, than idle ones gain, 1 of 8 of 4096 -> 14336 21.2 / 22.1.)
             int best = 0;
             double best_t = 0.0;
-            for (int sp = 1; sp <= blocks; ++sp)
+            const int nk_all = (g.indices || (g.size_n && !g.n_stride)) && mt <= 4 ? 8 : blocks;
+            for (int nk_max = nk_all; !best; nk_max = blocks)
             {
-                const int nk = (blocks + sp - 1) / sp;           // 128-row chunks of the longest range
-                if ((size_t) mt * (nk * 128 + 4) * 4 > (size_t) GEMVM_STAGED_X_BYTES) continue;
-                if ((size_t) sp * bszm * m * n * 4 > partial_bytes && sp > 1) break;
-                if (best && (long) bszm * chunks * sp > 8L * num_cus) break;     // only slower from here on
-                const long per = ((long) bszm * chunks * sp + num_cus - 1) / num_cus;     // workgroups of a CU
-                const double t = 2.0 + per * 0.5 * ((double) blocks / sp + nk) * (0.5 + 0.027 * m) * (per == 1 ? 1.65 : 1.0) + 0.5 * per
-                         + (sp > 1 ? 1.5 + 0.02 * m * sp : 0.0);
-                if (!best || t < best_t) { best = sp; best_t = t; }
+                for (int sp = 1; sp <= blocks; ++sp)
+                {
+                    const int nk = (blocks + sp - 1) / sp;       // 128-row chunks of the longest range
+                    if (nk > nk_max || (size_t) mt * (nk * 128 + 4) * 4 > (size_t) GEMVM_STAGED_X_BYTES) continue;
+                    if ((size_t) sp * bszm * m * n * 4 > partial_bytes && sp > 1) break;
+                    if (best && (long) bszm * chunks * sp > 8L * num_cus) break;     // only slower from here on
+                    const long per = ((long) bszm * chunks * sp + num_cus - 1) / num_cus;     // workgroups of a CU
+                    const double t = 2.0 + per * 0.5 * ((double) blocks / sp + nk) * (0.5 + 0.027 * m) * (per == 1 ? 1.65 : 1.0) + 0.5 * per
+                             + (sp > 1 ? 1.5 + 0.02 * m * sp : 0.0);
+                    if (!best || t < best_t) { best = sp; best_t = t; }
+                }
+                if (nk_max == blocks) break;
             }
             if (best > 0)
             {

@@ -134,3 +134,41 @@ def test_bundle_split_with_idle_slots(torch_cuda, kernel_policy, form):
         ops.exl3_mgemm(A, P(0, 2), C, P(1, 2), A_had, P(2, 2), idx, None, 4, min_index=lo, max_index=hi)
         return C[:2].clone()
     assert same_as_split(torch, kernel_policy, call, (16, 32)) == [True, False]
+
+
+@pytest.mark.parametrize("form", ["indices", "filter", "widths", "full"])
+@pytest.mark.parametrize("m", [2, 4])
+def test_rows_split_with_idle_slots(torch_cuda, orc, form, m):
+    """The same for 2 to 4 rows, where a range holds at most 8 chunks of 128 rows with lists: 9 chunks are split
+    (partial sums in the workspace), which 64 slots in use are not."""
+    from ampstein_amd import ops
+    torch = torch_cuda
+    if _device_cus() != 256:
+        pytest.skip("the sizes are for 256 CUs")
+    k, n, slots = 1152, 1536, 64
+    layers = [synth.layer(k, n, 4, 0, seed=9400 + i) for i in range(2)]
+    mats = [L.torch() for L in layers]
+    P = lambda i, num: ops.ptr_array([mats[j % 2][i] for j in range(num)])
+    x = synth.activations(m, k, seed=9401)
+    A = torch.from_numpy(x).cuda()[None]
+    A_had = torch.empty((slots, m, k), dtype=torch.half, device="cuda")
+    C = torch.zeros((slots, m, n), dtype=torch.float, device="cuda")
+    dev = torch.cuda.current_device()
+    _lib.check(_lib.lib().exl3_amd_debug_fill_workspace(dev, 0xFF))
+    if form == "widths":
+        widths = torch.tensor([n] + [128] * (slots - 1), dtype=torch.int32, device="cuda")
+        c_ptrs = ops.ptr_array([C.data_ptr() + j * m * n * 4 for j in range(slots)])
+        ops.exl3_mgemm(A, P(0, slots), C, P(1, slots), A_had, P(2, slots), None, None, 4, size_n_list=widths, c_ptrs=c_ptrs)
+    elif form == "full":
+        ops.exl3_mgemm(A, P(0, slots), C, P(1, slots), A_had, P(2, slots), None, None, 4)
+    else:
+        idx = torch.full((1, slots), -1 if form == "indices" else 1000, dtype=torch.long, device="cuda")
+        idx[0, 0], idx[0, 1] = 0, 1
+        lo, hi = (-1, -1) if form == "indices" else (0, 2)
+        ops.exl3_mgemm(A, P(0, 2), C, P(1, 2), A_had, P(2, 2), idx, None, 4, min_index=lo, max_index=hi)
+    torch.cuda.synchronize()
+    L = layers[0]
+    check(C[0], orc.linear_f64(x, L.trellis, L.suh, L.svh, 4, cb=0), (form, m))
+    head = np.empty(m * n, np.uint32)
+    _lib.check(_lib.lib().exl3_amd_debug_read_workspace(dev, 0, head.nbytes, head.ctypes.data))
+    assert bool((head != 0xFFFFFFFF).any()) == (form != "full")
