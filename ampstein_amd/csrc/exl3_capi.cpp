@@ -593,7 +593,10 @@ int dispatch_rows(int bits, int cb, const RowsArgs& g, hipStream_t s)
 
 // Row tiles and k split of the row-tile GEMM (exl3_rows.hip).  As few row tiles as 128 rows allow,
 // equal in height.  The k split S minimises this model (us, fitted on MI355X over K = 3 / 4, nine
-// shapes from 4096 x 1024 to 8192 x 28672 and S = 1..32; within ~10 %):
+// shapes from 4096 x 1024 to 8192 x 28672 and S = 1..32, to an earlier form of the kernel).  Against
+// the kernel as it is, over 14 shapes, K = 2 mul1, 4 and 8 and 9..512 rows, the S it takes costs 0.7 % on average over
+// the best of ten from 1 to 32, 15 % at worst (512 rows of 1024 x 4096: S = 2, best 1).  The time it gives is
+// too long: the kernel takes 0.8 of it at 1 to 2 row groups, 0.9 at 8, and 1.0 at 8 bits, which it does not know.
 //   rounds of workgroups over the CUs x units per k half (128 k each) x the unit's time, which the
 //   decode sets and the row groups add to; the fill and the epilogue once per round (twice as
 //   many workgroups share a CU up to 4 groups); the last arrival's sum of S partials per group.
@@ -1027,9 +1030,12 @@ int gemm_impl(const Workspace* ws, const uint16_t* A, const uint16_t* trellis, v
     const uint16_t* A_rot = suh ? A_had : A;
     // More than 8 rows: the row-tile GEMM (exl3_rows.hip), the tiled GEMM or, up to 16 rows, the
     // matrix-core GEMV, whichever its time model puts first (us, input rotation included).  Measured
-    // on MI355X (K = 4 3INST, row tiles / tiled GEMM): 4096 x 14336 at 33 / 100 / 256 rows 27 / 38 /
-    // 59 against 52 / 56 / 66, 17408 x 5120 37 / 52 / 87 against 68 / 71 / 83, 8192 x 28672 80 / 97
-    // / 209 against 152 / 154 / 174: row tiles up to ~128-250 rows, the tiled GEMM above.
+    // on MI355X (K = 4 3INST, row tiles / tiled GEMM): 4096 x 14336 at 24 / 100 / 256 rows 21 / 35 / 50
+    // against 50 / 55 / 65, 17408 x 5120 27 / 47 / 72 against 66 / 69 / 80, 8192 x 28672 50 / 83 / 162
+    // against 144 / 146 / 165.  The models do not know how fast the row tiles are by now: over 13 shapes, 10 bitrates
+    // and codebooks and 9 to 768 rows the choice costs 1.7 % on average over the best kernel, 54 % at worst (100 rows
+    // of 4096 x 1024: tiled 33, row tiles 22; the GEMV at 16 rows of 5120 x 5120: 19 against 14), and twice the
+    // time on deep narrow layers without the hand-off (200 rows of 8192 x 384: tiled 44, row tiles 22).
     //   tiled GEMM: 22 us + 30 ns per k of a round (of a split), and with the split k 0.25 us per MB
     //   of partial tiles; GEMV group: 8 us + 0.37 ns per 1000 weights.
     // force_shape_idx 1 takes the GEMV for any row count (16-row groups, each split in two
@@ -1504,9 +1510,12 @@ int exl3_amd_moe(const uint16_t* hidden_state, int bsz, int hidden_dim, float* o
                           hidden_dim <= DMA_MAX_K && intermediate_dim <= DMA_MAX_K;
     // moeg: the smallest tile holding ~1.5x the mean rows (the largest expert, for top-k routing
     // of random tokens).  Measured, 256 experts 4096 -> 2048 -> 4096, top-8: T = 512 (mean 16,
-    // max 27) best at 32 or 64 (0.99 / 1.07 ms); T = 1024 (mean 32) at 64: 1.19 against 1.48 at 32 and
-    // 1.35 at 96; T = 2048 (mean 64, max 91) at 96: 1.66 against 2.01 at 64 and 2.03 at 128 (fewer
-    // tiles decode each expert's weights fewer times; 96 keeps 3 waves per SIMD)
+    // max 27) best at 32 or 64 (0.89 / 0.94 ms); T = 1024 (mean 32) at 64: 1.06 against 1.35 at 32 and
+    // 1.21 at 96; T = 2048 (mean 64, max 91) at 96: 1.49 against 1.77 at 64 and 1.68 at 128 (fewer
+    // tiles decode each expert's weights fewer times; 96 keeps 3 waves per SIMD).  From a mean of 128 on 96
+    // and 128 are close: mean 128 / 256 at 96 against 128 rows, 256 experts 2.98 / - against 2.98 / - ms, 128
+    // experts 2048 -> 768 446 / 750 against 435 / 769 us, 64 experts 2048 -> 1536 371 / 606 against 359 / 632, 16 experts
+    // 3072 -> 1024 132 / 187 against 142 / 206 (mean 512: 327 against 321)
     const int want = mean_rows * 3 / 2;
     int tile_rows = reg_gemm ? (want <= 32 ? 32 : (want <= 64 ? 64 : (want <= 96 ? 96 : 128)))
                              : (mean_rows <= 40 ? 64 : (mean_rows <= 96 ? 128 : 256));

@@ -15,8 +15,8 @@
 //   B       the same GEMV over the down trellis; the last arrival of a (token, chunk) rotates
 //           each active slot's sum * svh (+ bias), weights it by its routing weight, sums the
 //           slots in the reference's fixed order (:917-999), adds the shared expert and stores.
-// A and B each launch once per run size class: single-slot runs with the one-row body (126
-// VGPRs, 4 waves per SIMD), larger runs with the eight-row body.  A token's slots can sit in
+// A and B each launch once per run size class: single-slot runs with the one-row body, larger runs with
+// the eight-row body (mul1: 103 and 127 VGPRs, 4 waves per SIMD).  A token's slots can sit in
 // both classes; its down hand-off counter then collects arrivals from both launches.
 //
 // Hand-offs: counters (one 128-byte line each) in the library workspace; chunk c runs on XCD
@@ -856,8 +856,9 @@ int EXL3_CAT(exl3k_moe_cb, EXL3_MOE_CB)(const MoeArgs& a, hipStream_t s)
     auto moe_lds_bytes = [](int mt) { return ((size_t) mt * (SBMAX * 16 + 4) + (size_t) NW * mt * 128 + (size_t) mt * 128) * 4; };
     const int rot_items = slots * (a.Hi / 128) * nproj;
     hipLaunchKernelGGL(moe_route_kernel, dim3((rot_items + NW - 1) / NW), dim3(NT), 0, s, a);
-    // Runs by size class, each with the GEMV body of its row count: VGPRs (126 for one row, 204
-    // for eight) set the waves per SIMD, and most runs of a decode batch hold a single slot.  A
+    // Runs by size class, each with the GEMV body of its row count (103 VGPRs for one row, 127 for eight with
+    // mul1): a single slot pays for one staged row and its dots only, and most runs of a decode batch
+    // hold one.  A
     // one-token batch has distinct picks but for repeats, so its single-row launch takes every
     // run (a repeat costs a second pass) and the eight-row launch is skipped.
     const int gridA = slots * (a.I / 128) * nproj * a.splits_a, gridB = slots * (a.Ho / 128) * a.splits_b;

@@ -38,10 +38,10 @@
 // once a unit, and at one rate the calls took 8 to 28 % longer at 2.5 bits, up to 34 % with few experts.
 //
 // What bounds it: the issue slots.  A unit is 96 VALU instructions of decode (bfe, mul, sad a weight)
-// per 10 MFMAs at 40 rows; the counters show 61 % of the cycles issuing VALU and 21 % in MFMAs, which
-// mostly add up.  So the products are made for the row groups that exist only (all four groups of a
-// 64-row tile always: 1.40 against 1.26 ms at 1024 tokens), while ring depth (2 or 4 units) and waves per
-// SIMD move the time by under 3 %.
+// per 10 MFMAs at 40 rows; of the cycles 81 % issue VALU and 17 % are in MFMAs at 512 tokens (256 experts 4096 ->
+// 2048, 32-row tiles), 67 and 41 % at 2048 (96-row tiles), and the two mostly add up.  So the products are
+// made for the row groups that exist only (all four groups of a 64-row tile always: 1.40 against 1.26 ms
+// at 1024 tokens, before the waits above).
 #include "exl3_common.cuh"
 #include "exl3_gemv_core.cuh"
 #include "exl3_kernels.h"

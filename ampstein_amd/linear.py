@@ -24,10 +24,12 @@ import torch
 from . import bundles, ops
 from .weights import Weights
 
-# exl3_gemm / exl3_gemm_recon on MI355X, us: 4096 -> 4096 at 145 / 256 / 512 rows 25 / 33 / 46
-# against 57 / 65 / 58, 14336 -> 4096 49 / 62 / 99 against 82 / 92 / 107, 8192 -> 28672 157 / 174 /
-# 296 against 250 / 246 / 324; at 768 rows of 17408 -> 5120 196 against 186, 8192 -> 28672 559
-# against 512.  exl3_gemm also needs no k x n fp16 buffer.
+# exl3_gemm / exl3_gemm_recon on MI355X, us, at 4 bits: 4096 -> 4096 at 145 / 256 / 512 rows 24 / 32 / 43
+# against 54 / 63 / 60, 14336 -> 4096 46 / 60 / 101 against 86 / 96 / 113, 8192 -> 28672 173 / 180 /
+# 324 against 248 / 250 / 325; at 768 rows of 17408 -> 5120 197 against 195, 8192 -> 28672 612
+# against 516 (but 4096 -> 4096 57 against 78).  Over 13 shapes and 10 bitrates and codebooks up to 512 rows
+# exl3_gemm is the slower one only for 5120 -> 17408 at 8 bits (512 rows: 190 against 178).  It also needs
+# no k x n fp16 buffer.
 RECON_ROWS = 512
 ENGINE_RECON_ROWS = 144   # models.uc:35
 RECON_MAX_N = 32768       # models.uc:36
